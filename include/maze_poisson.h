@@ -269,6 +269,13 @@ void maze_test_laplace_pb(const double *u, double *out, int n, const double *eps
 int maze_test_conj_grad(const double *b, double *x, double tol, int n);
 int maze_test_conj_grad_pb(const double *b, double *x, double tol, int n, const double *eps_x,
                            const double *eps_y, const double *eps_z, const double *k2);
+/* The same solves (ex == NULL: Poisson) with one or two reductions per
+ * iteration, as sweeps (onchip 0) or as one launch with the CG vectors on the
+ * chip (bit-identical; -2 if the grid does not fit it, -3 if the launch was
+ * abandoned and the sweeps ran; onchip 2: it starts abandoned). */
+int maze_test_conj_grad_form(const double *b, double *x, double tol, int n, const double *eps_x,
+                             const double *eps_y, const double *eps_z, const double *k2,
+                             int reductions, int onchip);
 void maze_test_rbgs(const double *in, double *out, int n, int iters);
 int maze_test_restrict27(const double *in, double *out, int n);
 int maze_test_prolong_add(const double *in, double *out, int nc);
@@ -320,7 +327,7 @@ int maze_test_mg_tail(const float *b, float *d, int n);
  * blocks until the solve has finished.  No counterpart in the reference: for
  * callers that cannot allocate device memory (code around graph captures,
  * tight serving loops, harnesses that forbid hipMalloc).  Its work space is one
- * statically allocated device array per GPU (6.4 MB, held until the process
+ * statically allocated device array per GPU (6.5 MB, held until the process
  * ends): grids of at most 64^3 points.  Calls that overlap on one GPU share
  * that array and race; serialise them.  Returns the 0-based iteration index
  * at convergence, -1 if not converged in n^2 iterations, -2 for n outside

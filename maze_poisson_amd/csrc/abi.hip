@@ -17,7 +17,10 @@ using maze::Sim;
 static Sim* g_sim = nullptr;
 
 static Sim& S() {
-    if (!g_sim) g_sim = new Sim();
+    if (!g_sim) {
+        g_sim = new Sim();
+        g_sim->onchip = 1;
+    }
     return *g_sim;
 }
 
@@ -366,31 +369,46 @@ void maze_test_laplace_pb(const double* u, double* out, int n, const double* ex,
     delete s;
 }
 
-int maze_test_conj_grad(const double* b, double* x, double tol, int n) {
+// FP64 CG with one or two reductions per iteration, as sweeps or in one launch
+// with its vectors on the chip (-2 where the grid does not fit, -3 if the launch
+// was abandoned and the sweeps ran).  ex == nullptr: the Poisson operator.
+int maze_test_conj_grad_form(const double* b, double* x, double tol, int n, const double* ex,
+                             const double* ey, const double* ez, const double* k2, int reductions,
+                             int onchip) {
     Sim* s = scratch_sim(n);
-    MAZE_HIP(hipMemcpy(s->sigma, b, s->G * sizeof(double), hipMemcpyHostToDevice));
-    MAZE_HIP(hipMemcpy(s->y, x, s->G * sizeof(double), hipMemcpyHostToDevice));
-    int pred = 32;
-    const int res = s->cg_solve(s->dims, maze::PBCoef{}, s->sigma, s->y, tol, n * n, s->r, s->p0,
-                                s->p1, &pred);
-    MAZE_HIP(hipMemcpy(x, s->y, s->G * sizeof(double), hipMemcpyDeviceToHost));
+    s->onchip = onchip != 0;
+    if (ex) {
+        s->init_pb(0.0, 0.0);
+        s->set_eps_k2(ex, ey, ez, k2);
+    }
+    s->precision = reductions == 2 ? maze::kMixedMG : maze::kFP64;
+    s->tol = tol;
+    int res = -2;
+    if (!onchip || (s->cg_two() ? maze::cg_onchip2_fits(s->dims) : maze::cg_onchip_fits(s->cgd))) {
+        MAZE_HIP(hipMemcpy(s->sigma, b, s->G * sizeof(double), hipMemcpyHostToDevice));
+        MAZE_HIP(hipMemcpy(s->y, x, s->G * sizeof(double), hipMemcpyHostToDevice));
+        int pred = 32;
+        if (onchip == 2) {
+            s->onchip_next(s->cg_two() ? s->dims : s->cgd, n * n, s->cg_two());
+            const unsigned int given_up = 1u << 30;
+            MAZE_HIP(hipMemcpy(s->onchip_w.ctl, &given_up, sizeof(given_up), hipMemcpyHostToDevice));
+            s->onchip_void = 1;
+        }
+        res = s->cg_solve(s->cg_run(s->y, s->sigma, pred + 1, &pred));
+        MAZE_HIP(hipMemcpy(x, s->y, s->G * sizeof(double), hipMemcpyDeviceToHost));
+        if (onchip && !s->onchip) res = -3;
+    }
     delete s;
     return res;
 }
 
+int maze_test_conj_grad(const double* b, double* x, double tol, int n) {
+    return maze_test_conj_grad_form(b, x, tol, n, nullptr, nullptr, nullptr, nullptr, 1, 0);
+}
+
 int maze_test_conj_grad_pb(const double* b, double* x, double tol, int n, const double* ex,
                            const double* ey, const double* ez, const double* k2) {
-    Sim* s = scratch_sim(n);
-    s->init_pb(0.0, 0.0);
-    s->set_eps_k2(ex, ey, ez, k2);
-    MAZE_HIP(hipMemcpy(s->sigma, b, s->G * sizeof(double), hipMemcpyHostToDevice));
-    MAZE_HIP(hipMemcpy(s->y, x, s->G * sizeof(double), hipMemcpyHostToDevice));
-    int pred = 32;
-    const int res = s->cg_solve(s->dims, s->pbc(), s->sigma, s->y, tol, n * n, s->r, s->p0, s->p1,
-                                &pred);
-    MAZE_HIP(hipMemcpy(x, s->y, s->G * sizeof(double), hipMemcpyDeviceToHost));
-    delete s;
-    return res;
+    return maze_test_conj_grad_form(b, x, tol, n, ex, ey, ez, k2, 1, 0);
 }
 
 void maze_test_rbgs(const double* in, double* out, int n, int iters) {

@@ -147,6 +147,42 @@ __device__ __forceinline__ double wave_max(double v) {
     return v;
 }
 
+// The same sums and maxima over the lanes with DPP moves: four exchanges inside
+// the rows of 16 lanes, then the rows' results as scalars.  The butterflies
+// above go through the LDS crossbar, about 100 cycles a step; these take
+// about 10.  (Another order of additions than wave_sum.)  All lanes active.
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+__device__ __forceinline__ double lane_value(double v, int l) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)b, l);
+    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140,
+              kDppRor8 = 0x128, kDppReverse4 = 0x1B;
+
+__device__ __forceinline__ double wave_sum_dpp(double v) {
+    v += dpp_move<kDppXor1>(v);
+    v += dpp_move<kDppXor2>(v);
+    v += dpp_move<kDppHalfMirror>(v);
+    v += dpp_move<kDppMirror>(v);
+    return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
+}
+
+__device__ __forceinline__ double wave_max_dpp(double v) {
+    v = fmax(v, dpp_move<kDppXor1>(v));
+    v = fmax(v, dpp_move<kDppXor2>(v));
+    v = fmax(v, dpp_move<kDppHalfMirror>(v));
+    v = fmax(v, dpp_move<kDppMirror>(v));
+    return fmax(fmax(lane_value(v, 0), lane_value(v, 16)), fmax(lane_value(v, 32), lane_value(v, 48)));
+}
+
 // Fixed-shape work-group reductions (deterministic: butterfly within each
 // wave, then the NT/64 wave results in wave order).  Result valid in all
 // threads; sh holds NT/64 doubles.
@@ -224,12 +260,13 @@ constexpr int kArrivalStride = 32;
 constexpr int kArrivalGroups = 8;
 constexpr int kArrivalWords = (kArrivalGroups + 1) * kArrivalStride;
 
-__device__ __forceinline__ bool publish_arrive(double* psum, double s, double* pmax, double m,
-                                               unsigned int* counter, unsigned int nblocks) {
+// store: called by thread 0, stores the work-group's partials (store_partial).
+template <class Store>
+__device__ __forceinline__ bool publish_arrive(Store&& store, unsigned int* counter,
+                                               unsigned int nblocks) {
     __shared__ bool last;
     if (threadIdx.x == 0) {
-        store_partial(psum, blockIdx.x, s);
-        if (pmax) store_partial(pmax, blockIdx.x, m);
+        store();
         __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
         const unsigned int g = blockIdx.x % kArrivalGroups;
         const unsigned int groups = nblocks < kArrivalGroups ? nblocks : kArrivalGroups;
@@ -246,6 +283,16 @@ __device__ __forceinline__ bool publish_arrive(double* psum, double s, double* p
     }
     __syncthreads();
     return last;
+}
+
+__device__ __forceinline__ bool publish_arrive(double* psum, double s, double* pmax, double m,
+                                               unsigned int* counter, unsigned int nblocks) {
+    return publish_arrive(
+        [&] {
+            store_partial(psum, blockIdx.x, s);
+            if (pmax) store_partial(pmax, blockIdx.x, m);
+        },
+        counter, nblocks);
 }
 
 // Zeroes the counters of publish_arrive (called by the last work-group, when

@@ -107,7 +107,7 @@ static int precision_for(int n, int want, const Phys& ph) {
 static long long arena_bytes(int n, int np, int precision, const Phys& ph) {
     const long long G = (long long)n * n * n;
     // reduction partials of both streams and of the deferred inner iteration, scalars
-    long long b = 8LL * 8 * (1 << 15) + (64 << 10);
+    long long b = (7LL + kCg1Sums) * 8 * (1 << 15) + (64 << 10);
     int allocs = 64;
     b += 9 * 8 * G;                                   // q, y, phi, phi_prev, phi*, sigma, r, p0, p1
     if (ph.grid_type == kMG || ph.grid_type == kMazeMG ||

@@ -84,6 +84,10 @@ struct Reduce {
     unsigned int* counter;
 };
 
+// The launch shape of the grid passes of an n^3 grid (planes per work-group
+// sized for about 512 work-groups per sweep); every replica uses it.
+GridDims grid_dims_for(int n);
+
 // ---- launchers (grid_kernels.hip) ----------------------------------------
 void launch_laplace(hipStream_t s, const GridDims& d, const PBCoef& pb, const double* u, double* out);
 void launch_pred_sigma(hipStream_t s, const GridDims& d, const PBCoef& pb, const double* phi,
@@ -106,8 +110,46 @@ void launch_cg_update(hipStream_t s, const GridDims& d, const PBCoef& pb, const 
 void launch_dot_rv(hipStream_t s, const GridDims& d, const double* r, const double* v, CGState* st,
                    Reduce red, int first);
 // gated: the solve is started only while the outer refinement loop runs.
+// meet: a counter word to zero (CgOnchip::ctl).
 void launch_cg_reset(hipStream_t s, CGState* st, double tol, double rtol, int limit, int count_mode,
-                     int pcg = 0, int gated = 0, int plain = 0);
+                     int pcg = 0, int gated = 0, int plain = 0, unsigned int* meet = nullptr);
+
+// FP64 CG with one reduction per iteration (Cg1, stencil.hpp), after
+// launch_cg_reset and launch_cg_init: launch_cg1_dir (the direction, A p, the
+// stop test of the update before it, alpha and the next beta), then
+// launch_cg1_update.  A solve of k updates ends in the direction pass after the
+// last.  red.psum: kCg1Sums partials per work-group.
+constexpr int kCg1Sums = 4;
+void launch_cg1_dir(hipStream_t s, const GridDims& d, const PBCoef& pb, const double* p_old,
+                    const double* r, double* p_new, CGState* st, Reduce red, int first);
+void launch_cg1_update(hipStream_t s, const GridDims& d, const PBCoef& pb, const double* p,
+                       double* x, double* r, CGState* st);
+
+// The same solve in one launch with its vectors on the chip (cg_onchip.hip),
+// after launch_cg_reset (which zeroes ctl) and launch_cg_init: the same bits in
+// x and st as those sweeps.  Its work-groups wait for each other, so the launch
+// needs the GPU's CUs to itself or beside kernels that end by themselves: no
+// two such launches at once.  A solve whose wait runs out leaves x and st
+// (st->done == 0) as they were.
+// h0, h1: scratch grids; words: cg_onchip_words() of them, zeroed once; epoch:
+// advances by more than the iterations + 2 per launch, words zeroed again
+// before it wraps.
+struct CgOnchip {
+    unsigned long long* words;
+    unsigned int* ctl;
+    unsigned int epoch;
+};
+// The launch shape of FP64 CG on an n^3 grid, in either form.
+GridDims cg_dims_for(int n);
+bool cg_onchip_fits(const GridDims& d);
+// launch_cg_dir / launch_cg_update's solve (two reductions an iteration) likewise,
+// h: one scratch grid; twice the epochs.
+bool cg_onchip2_fits(const GridDims& d);
+void launch_cg_onchip2(hipStream_t s, const GridDims& d, const PBCoef& pb, double* x, double* r,
+                       double* h, CGState* st, const CgOnchip& w);
+long cg_onchip_words();
+void launch_cg_onchip(hipStream_t s, const GridDims& d, const PBCoef& pb, double* x, double* r,
+                      double* h0, double* h1, CGState* st, const CgOnchip& w);
 
 // Mixed precision, FP64 true residual of the refinement loop, b = sigma - A y.
 // First pass (add_d == 0): y = y0, starts the loop (ysel = 0).

@@ -293,6 +293,138 @@ void launch_cg_update32(hipStream_t s, const GridDims& d, const PBCoef32& pb, co
                     s, d, pb, p, x, r, red, st);
 }
 
+// ---- CG with one reduction per iteration (Cg1) -----------------------------------
+// The update no longer ends in a reduction, and the direction pass reads r's
+// centre value, which its source loads anyway.
+struct BodyDir1 {
+    double* p_new;
+    const double* r;
+    double s[kCg1Sums] = {0.0, 0.0, 0.0, 0.0}, m = 0.0;
+    using Raw = double;
+    __device__ Raw load(int c) const { return r[c]; }
+    __device__ void apply(int c, const Raw& rc, double v, double lap) {
+        p_new[c] = v;
+        cg1_terms(v, rc, lap, s, m);
+    }
+};
+
+struct BodyUpdate1 {
+    double* x;
+    double* r;
+    double alpha;
+    struct Raw { double x, r; };
+    __device__ Raw load(int c) const { return Raw{x[c], r[c]}; }
+    __device__ void apply(int c, const Raw& o, double v, double lap) {
+        x[c] = o.x + alpha * v;
+        r[c] = o.r + alpha * lap;
+    }
+};
+
+// Partials by tile, not by work-group id: value c of tile b at psum[c nb + b].
+// The last work-group adds the tiles of neighbouring plane chunks in pairs
+// (what one work-group of the on-chip form holds), folds the pairs in groups of
+// 64 (one wave each), then the groups in order.
+constexpr int kCg1Groups = (1 << 15) / kWave;  // of the largest launch
+
+template <bool PB, bool First>
+__global__ __launch_bounds__(kBlock) void k_cg1_dir(GridDims d, PBCoef pb, const double* p_old,
+                                                    const double* r, double* p_new, Reduce red,
+                                                    CGState* st) {
+    if (st->done) return;
+    constexpr int NW = kBlock / kWave, NV = kCg1Sums + 1;
+    __shared__ double sh[NV][NW], shg[kCg1Groups * NV], tot[NV];
+    const SrcDir<double, First> src{p_old, r, First ? 0.0 : st->beta, st->plain ? -1.0 : 1.0 / 6.0};
+    BodyDir1 bd{p_new, r};
+    march<PB>(d, pb, src, bd);
+    const int t = threadIdx.x, lane = t & (kWave - 1), w = t / kWave, nb = gridDim.x;
+    const int tile = xcd_tile(blockIdx.x, nb);
+#pragma unroll
+    for (int c = 0; c < kCg1Sums; c++) bd.s[c] = wave_sum_dpp(bd.s[c]);
+    bd.m = wave_max_dpp(bd.m);
+    if (lane == 0) {
+#pragma unroll
+        for (int c = 0; c < kCg1Sums; c++) sh[c][w] = bd.s[c];
+        sh[kCg1Sums][w] = bd.m;
+    }
+    __syncthreads();
+    const bool last = publish_arrive(
+        [&] {
+#pragma unroll
+            for (int c = 0; c < kCg1Sums; c++) store_partial(red.psum, c * nb + tile, cg1_tile(sh[c]));
+            store_partial(red.pmax, tile, cg1_pair_max(sh[kCg1Sums], sh[kCg1Sums]));
+        },
+        red.counter, nb);
+    if (!last) return;
+    const int per = (d.chunks + 1) / 2, pairs = per * d.slabs, J = (pairs + kWave - 1) / kWave;
+    const int val = lane & 7, vc = min(val, kCg1Sums);
+    const double* part = vc < kCg1Sums ? red.psum + vc * nb : red.pmax;
+    for (int g = w; g < J; g += NW) {
+        double v[8], u[8];
+        bool two[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int pc = min(g * kWave + 8 * i + lane / 8, pairs - 1);
+            const int s = pc / per, ch = 2 * (pc - s * per), a = s * d.chunks + ch;
+            two[i] = ch + 1 < d.chunks;
+            v[i] = load_partial(part, a);
+            u[i] = load_partial(part, two[i] ? a + 1 : a);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            v[i] = vc < kCg1Sums ? v[i] + (two[i] ? u[i] : 0.0) : fmax(v[i], u[i]);
+            if (g * kWave + 8 * i + lane / 8 >= pairs) v[i] = 0.0;
+        }
+        const double f = cg1_fold(v, vc == kCg1Sums);
+        if (lane < NV) shg[g * NV + lane] = f;
+    }
+    __syncthreads();
+    if (t < NV) {
+        double v = shg[t];
+        for (int g = 1; g < J; g++) v = t < kCg1Sums ? v + shg[g * NV + t] : fmax(v, shg[g * NV + t]);
+        tot[t] = v;
+    }
+    __syncthreads();
+    if (t != 0) return;
+    Cg1 cg;
+    int res = -1;
+    const int it = st->iter;
+    const bool stop = cg.decide(tot, tot[kCg1Sums], it, st->limit, st->count_mode, st->plain,
+                                st->tol, st->rtol * st->r0, res);
+    cg.store(st);
+    if (stop) {
+        st->res = res;
+        st->done = 1;
+    } else {
+        st->iter = it + 1;
+    }
+    reset_arrivals(red.counter);
+}
+
+template <bool PB>
+__global__ __launch_bounds__(kBlock) void k_cg1_update(GridDims d, PBCoef pb, const double* p,
+                                                       double* x, double* r, const CGState* st) {
+    if (st->done) return;
+    BodyUpdate1 bd{x, r, st->alpha};
+    march<PB>(d, pb, SrcArr<double>{p}, bd);
+}
+
+void launch_cg1_dir(hipStream_t s, const GridDims& d, const PBCoef& pb, const double* p_old,
+                    const double* r, double* p_new, CGState* st, Reduce red, int first) {
+    if (first) {
+        DISPATCH_PB(pb, MAZE_LAUNCH((k_cg1_dir<kPB, true>), dim3(d.blocks), dim3(kBlock), 0, s, d,
+                                    pb, p_old, r, p_new, red, st));
+    } else {
+        DISPATCH_PB(pb, MAZE_LAUNCH((k_cg1_dir<kPB, false>), dim3(d.blocks), dim3(kBlock), 0, s, d,
+                                    pb, p_old, r, p_new, red, st));
+    }
+}
+
+void launch_cg1_update(hipStream_t s, const GridDims& d, const PBCoef& pb, const double* p,
+                       double* x, double* r, CGState* st) {
+    DISPATCH_PB(pb, MAZE_LAUNCH((k_cg1_update<kPB>), dim3(d.blocks), dim3(kBlock), 0, s, d, pb, p, x,
+                                r, st));
+}
+
 template void launch_cg_init<double>(hipStream_t, const GridDims&, const PBCoef&, const double*,
                                      const double*, double*, CGState*, Reduce, double*, int);
 template void launch_cg_init<float>(hipStream_t, const GridDims&, const PBCoef&, const float*,
@@ -313,8 +445,9 @@ void launch_dot_rv(hipStream_t s, const GridDims& d, const double* r, const doub
 }
 
 __global__ void k_cg_reset(CGState* st, double tol, double rtol, int limit, int count_mode,
-                           int pcg, int gated, int plain) {
+                           int pcg, int gated, int plain, unsigned int* meet) {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
+        if (meet) *meet = 0u;
         if (gated && st->outer_done) {
             st->done = 1;
             return;
@@ -333,9 +466,9 @@ __global__ void k_cg_reset(CGState* st, double tol, double rtol, int limit, int 
 }
 
 void launch_cg_reset(hipStream_t s, CGState* st, double tol, double rtol, int limit,
-                     int count_mode, int pcg, int gated, int plain) {
+                     int count_mode, int pcg, int gated, int plain, unsigned int* meet) {
     MAZE_LAUNCH(k_cg_reset, dim3(1), dim3(64), 0, s, st, tol, rtol, limit, count_mode, pcg, gated,
-                plain);
+                plain, meet);
 }
 
 // The y buffers are chosen on the device (st->ysel), so a queued pass needs

@@ -25,7 +25,7 @@ constexpr size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 constexpr size_t kOffState = 0;
 constexpr size_t kOffCounter = align256(kOffState + sizeof(CGState));
 constexpr size_t kOffPsum = align256(kOffCounter + kArrivalWords * sizeof(unsigned int));
-constexpr size_t kOffPmax = align256(kOffPsum + kNoAllocMaxPartials * sizeof(double));
+constexpr size_t kOffPmax = align256(kOffPsum + kCg1Sums * kNoAllocMaxPartials * sizeof(double));
 constexpr size_t kOffR = align256(kOffPmax + kNoAllocMaxPartials * sizeof(double));
 constexpr size_t kOffP0 = align256(kOffR + kNoAllocMaxG * sizeof(double));
 constexpr size_t kOffP1 = align256(kOffP0 + kNoAllocMaxG * sizeof(double));
@@ -79,7 +79,7 @@ extern "C" int maze_conj_grad_noalloc(const double* b, double* x, double tol, in
         std::fprintf(stderr, "maze_conj_grad_noalloc: b and x must be device pointers\n");
         return -2;
     }
-    const GridDims d = grid_dims_for(n);
+    const GridDims d = cg_dims_for(n);
     if (d.blocks > kNoAllocMaxPartials) {
         std::fprintf(stderr, "maze_conj_grad_noalloc: %d work-groups exceed the %ld partials\n",
                      d.blocks, kNoAllocMaxPartials);
@@ -105,14 +105,15 @@ extern "C" int maze_conj_grad_noalloc(const double* b, double* x, double tol, in
     int launched = 0, chunk = 33;
     CGState h{};
     for (;;) {
-        for (int c = 0; c < chunk && launched < limit; c++, launched++) {
-            launch_cg_dir<double>(s, d, PBCoef{}, pa, r, pb, st, red, launched == 0);
-            launch_cg_update<double>(s, d, PBCoef{}, pb, x, r, st, red);
+        // (The direction pass after update `limit` applies its stop test.)
+        for (int c = 0; c < chunk && launched <= limit; c++, launched++) {
+            launch_cg1_dir(s, d, PBCoef{}, pa, r, pb, st, red, launched == 0);
+            launch_cg1_update(s, d, PBCoef{}, pb, x, r, st);
             std::swap(pa, pb);
         }
         MAZE_HIP(hipMemcpyAsync(&h, st, sizeof(CGState), hipMemcpyDeviceToHost, s));
         MAZE_HIP(hipStreamSynchronize(s));
-        if (h.done || launched >= limit) break;
+        if (h.done || launched > limit) break;
         chunk = std::max(4, chunk / 4);
     }
     return h.res;

@@ -129,7 +129,7 @@ Sim::Sim(hipStream_t main, hipStream_t side_) {
     st_c = dalloc<CGState>(1);
     MAZE_HIP(hipHostMalloc(&st_host, sizeof(CGState)));
     std::memset(st_host, 0, sizeof(CGState));
-    red.psum = dalloc<double>(kMaxPartials);
+    red.psum = dalloc<double>((long)kCg1Sums * kMaxPartials);
     red.pmax = dalloc<double>(kMaxPartials);
     red.counter = dalloc<unsigned int>(kArrivalWords);
     dred.pz = dalloc<double>(kMaxPartials);
@@ -167,6 +167,8 @@ Sim::~Sim() {
     dfree(red_side.counter);
     dfree(dscalar);
     dfree(ps);
+    dfree(onchip_w.words);
+    dfree(onchip_w.ctl);
     if (st_host) MAZE_HIP(hipHostFree(st_host));
     if (hscalar) MAZE_HIP(hipHostFree(hscalar));
     if (ps_host) MAZE_HIP(hipHostFree(ps_host));
@@ -247,6 +249,7 @@ void Sim::init_grid(int n_, double L_, double h_, double tol_, double eps, doubl
     pb = 0;
     G = (long)n * n * n;
     dims = grid_dims_for(n);
+    cgd = cg_dims_for(n);
     if (dims.blocks > kMaxPartials) fatal("maze: grid too large for the reduction buffers");
     q = dalloc<double>(G); y = dalloc<double>(G); phi = dalloc<double>(G);
     spread_zero_old = 0;
@@ -254,7 +257,7 @@ void Sim::init_grid(int n_, double L_, double h_, double tol_, double eps, doubl
     r = dalloc<double>(G); p0 = dalloc<double>(G); p1 = dalloc<double>(G);
     if (type == kMG || type == kMazeMG || (type == kMazeLCG && precond_ == kPMG)) {
         nc = n / 2;
-        cdims = make_dims(nc, choose_slab(nc));
+        cdims = cg_dims_for(nc);
         const long Gc = (long)nc * nc * nc;
         mg_r = dalloc<double>(G);
         if (type == kMazeLCG) pv = dalloc<double>(G);
@@ -536,29 +539,69 @@ void Sim::prof_flush_passes(const int* iters, int npass) {
 // Implicit-Jacobi CG, library/src/plcg.c:28-90: x holds the warm start.
 // Iterations are launched in chunks sized from the previous solve and the
 // device-side stop flag is polled between chunks.
-int Sim::cg_solve(const GridDims& d, const PBCoef& pbc_, const double* b, double* x, double tol_,
-                  int limit, double* rbuf, double* pa, double* pbuf, int* pred) {
-    cg_issue(CgRun{d, pbc_, x, rbuf, pa, pbuf, limit, 0, std::max(4, *pred + 1), pred}, b, tol_);
+int Sim::cg_solve(const CgRun& c) {
+    cg_issue(c);
     return cg_finish();
 }
 
-// The first chunk of a CG solve, up to the publication of its state.
-void Sim::cg_issue(const CgRun& c, const double* b, double tol_) {
+// A CG solve up to the publication of its state: whole (on the chip), or its
+// first chunk of iterations.
+void Sim::cg_issue(const CgRun& c) {
     cg = c;
-    launch_cg_reset(stream, st, tol_, 0.0, cg.limit, 0);
-    launch_cg_init<double>(stream, cg.d, cg.pbc, cg.x, b, cg.rbuf, st, red);
-    cg_chunk();
+    cg.onchip = onchip_next(cg.d, cg.limit, cg.two);
+    cg_start();
+    if (!cg.onchip)
+        cg_chunk();
+    else if (cg.two)
+        launch_cg_onchip2(stream, cg.d, cg.pbc, cg.x, cg.rbuf, cg.pin, st, onchip_w);
+    else
+        launch_cg_onchip(stream, cg.d, cg.pbc, cg.x, cg.rbuf, cg.pin, cg.pout, st, onchip_w);
     publish();
 }
 
+void Sim::cg_start() {
+    launch_cg_reset(stream, st, cg.tol, 0.0, cg.limit, 0, 0, 0, 0,
+                    onchip_void ? nullptr : onchip_w.ctl);
+    launch_cg_init<double>(stream, cg.d, cg.pbc, cg.x, cg.b, cg.rbuf, st, red);
+}
+
+bool Sim::onchip_next(const GridDims& d, int limit, int two) {
+    // Per-kernel timing names the sweeps, so it runs them.
+    if (!onchip || prof || !(two ? cg_onchip2_fits(d) : cg_onchip_fits(d))) return false;
+    const long words = cg_onchip_words();
+    const unsigned int span = 2u * (unsigned int)limit + 4u;
+    if (!onchip_w.words) {
+        onchip_w.words = dalloc<unsigned long long>(words);
+        onchip_w.ctl = dalloc<unsigned int>(1);
+        onchip_w.epoch = 1u;
+    } else if (onchip_w.epoch > 0xffffffffu - 2u * span) {
+        launch_fill(stream, words, 0.0, reinterpret_cast<double*>(onchip_w.words));
+        onchip_w.epoch = 1u;
+    } else {
+        onchip_w.epoch += onchip_span;
+    }
+    onchip_span = span;
+    return true;
+}
+
+// With one reduction, the direction pass after update `limit` applies its stop test.
 void Sim::cg_chunk() {
-    for (int c = 0; c < cg.chunk && cg.launched < cg.limit; c++, cg.launched++) {
+    for (int c = 0; c < cg.chunk && cg.launched < cg.limit + (cg.two ? 0 : 1);
+         c++, cg.launched++) {
         const int it = cg.launched;
         timed(kTCgDir, it, [&] {
-            launch_cg_dir<double>(stream, cg.d, cg.pbc, cg.pin, cg.rbuf, cg.pout, st, red, it == 0);
+            if (cg.two)
+                launch_cg_dir<double>(stream, cg.d, cg.pbc, cg.pin, cg.rbuf, cg.pout, st, red,
+                                      it == 0);
+            else
+                launch_cg1_dir(stream, cg.d, cg.pbc, cg.pin, cg.rbuf, cg.pout, st, red, it == 0);
         });
-        timed(kTCgUpdate, it,
-              [&] { launch_cg_update<double>(stream, cg.d, cg.pbc, cg.pout, cg.x, cg.rbuf, st, red); });
+        timed(kTCgUpdate, it, [&] {
+            if (cg.two)
+                launch_cg_update<double>(stream, cg.d, cg.pbc, cg.pout, cg.x, cg.rbuf, st, red);
+            else
+                launch_cg1_update(stream, cg.d, cg.pbc, cg.pout, cg.x, cg.rbuf, st);
+        });
         std::swap(cg.pin, cg.pout);
     }
 }
@@ -566,12 +609,20 @@ void Sim::cg_chunk() {
 // Waits for the published state; further chunks until the stop.
 int Sim::cg_finish() {
     wait_published();
-    while (!st_host->done && cg.launched < cg.limit) {
+    if (cg.onchip) {
+        if (!st_host->done) {  // abandoned: x is untouched, the sweeps run the solve
+            onchip = cg.onchip = 0;
+            cg_start();
+            cg_chunk();
+            read_state();
+        }
+    }
+    while (!st_host->done && cg.launched < cg.limit + (cg.two ? 0 : 1)) {
         cg.chunk = std::max(4, cg.chunk / 4);
         cg_chunk();
         read_state();
     }
-    const int done_iters = st_host->res >= 0 ? st_host->res + 1 : cg.launched;
+    const int done_iters = st_host->res >= 0 ? st_host->res + 1 : cg.limit;
     prof_flush(done_iters);
     *cg.pred = done_iters;
     return st_host->res;
@@ -585,6 +636,17 @@ int Sim::cg_count_solve(const GridDims& d, const PBCoef& cpb, const double* b, d
                         double rtol, int maxit, double* rbuf, double* pa, double* pbuf, int* pred,
                         CGState* st) {
     const int plain = cpb.ex ? 1 : 0;
+    if (onchip_next(d, maxit)) {
+        launch_cg_reset(stream, st, 0.0, rtol, maxit, 1, 0, 0, plain, onchip_w.ctl);
+        launch_cg_init<double>(stream, d, cpb, x, b, rbuf, st, red, nullptr, plain);
+        launch_cg_onchip(stream, d, cpb, x, rbuf, pa, pbuf, st, onchip_w);
+        read_state(st);
+        if (st_host->done) {
+            *pred = std::max(1, st_host->res);
+            return st_host->res;
+        }
+        onchip = 0;  // abandoned: x is untouched
+    }
     launch_cg_reset(stream, st, 0.0, rtol, maxit, 1, 0, 0, plain);
     launch_cg_init<double>(stream, d, cpb, x, b, rbuf, st, red, nullptr, plain);
     int launched = 0;
@@ -592,13 +654,13 @@ int Sim::cg_count_solve(const GridDims& d, const PBCoef& cpb, const double* b, d
     double* pin = pa;
     double* pout = pbuf;
     for (;;) {
-        for (int c = 0; c < chunk && launched < maxit; c++, launched++) {
-            launch_cg_dir<double>(stream, d, cpb, pin, rbuf, pout, st, red, launched == 0);
-            launch_cg_update<double>(stream, d, cpb, pout, x, rbuf, st, red);
+        for (int c = 0; c < chunk && launched <= maxit; c++, launched++) {
+            launch_cg1_dir(stream, d, cpb, pin, rbuf, pout, st, red, launched == 0);
+            launch_cg1_update(stream, d, cpb, pout, x, rbuf, st);
             std::swap(pin, pout);
         }
         read_state(st);
-        if (st_host->done || launched >= maxit) break;
+        if (st_host->done || launched > maxit) break;
         chunk = std::max(4, chunk / 4);
     }
     *pred = std::max(1, st_host->res);
@@ -1015,8 +1077,7 @@ void Sim::fp64_issue() {
     phip = phi;
     phi = tmp;
     tmp = old_phip;
-    cg_issue(CgRun{dims, pbc(), y, r, p0, p1, n * n, 0, std::max(4, last_iters + 1), &last_iters},
-             sigma, tol);
+    cg_issue(cg_run(y, sigma, std::max(4, last_iters + 1), &last_iters));
 }
 
 int Sim::fp64_finish() {
@@ -1261,7 +1322,7 @@ int Sim::lcg_update() {
     if (!pb) c /= eps_s;
     launch_copy(stream, G, phi, phip);
     launch_scale_copy(stream, G, c, q, y);
-    return cg_solve(dims, pbc(), y, phi, tol, n * n, r, p0, p1, &last_iters);
+    return cg_solve(cg_run(phi, y, std::max(4, last_iters + 1), &last_iters));
 }
 
 // Reference two-grid V-cycle, library/src/multigrid.c:99-168 (3 RBGS sweeps
@@ -1449,8 +1510,7 @@ void Sim::init_field_issue() {
         return;
     }
     cold_pred = std::max(32, last_iters);
-    cg_issue(CgRun{dims, pbc(), phi, r, p0, p1, n * n, 0, std::max(4, cold_pred + 1), &cold_pred},
-             sigma, tol);
+    cg_issue(cg_run(phi, sigma, std::max(4, cold_pred + 1), &cold_pred));
 }
 
 bool Sim::init_field_ready() const { return published(); }
@@ -1500,7 +1560,7 @@ void Sim::cold_finish() {
     if (st_host->ysel) launch_copy(stream, G, m.yb, phi);
     if (!converged) {  // finish with FP64 CG from the refined iterate
         int pred = std::max(32, last_iters);
-        cg_solve(dims, pbc(), sigma, phi, tol, n * n, r, p0, p1, &pred);
+        cg_solve(cg_run(phi, sigma, std::max(4, pred + 1), &pred));
     }
 }
 

@@ -54,10 +54,6 @@ struct KernelTimer {
     double bytes_per_launch = 0.0;
 };
 
-// The launch shape of the grid passes of an n^3 grid (planes per work-group
-// sized for about 512 work-groups per sweep); every replica uses it.
-GridDims grid_dims_for(int n);
-
 struct Sim {
     hipStream_t stream = nullptr;
 
@@ -93,6 +89,7 @@ struct Sim {
     double w = 0, kbar2 = 0;
     long G = 0;
     GridDims dims{};
+    GridDims cgd{};  // of the FP64 CG solves (cg_dims_for)
     double *q = nullptr, *y = nullptr, *phi = nullptr, *phip = nullptr, *tmp = nullptr;
     double *sigma = nullptr, *r = nullptr, *p0 = nullptr, *p1 = nullptr, *y_alt = nullptr;
     double* y_hist = nullptr;  // y of the step before last (extrapolated start)
@@ -192,7 +189,32 @@ struct Sim {
         double *pin, *pout;
         int limit, launched, chunk;
         int* pred;
+        const double* b;
+        double tol;
+        int two;     // two reductions per iteration (launch_cg_dir, launch_cg_update)
+        int onchip;  // the solve was queued as one launch (launch_cg_onchip)
     } cg{};
+    // FP64 CG solves in one launch with their vectors on the chip where the grid
+    // fits (cg_onchip_fits) -- for replicas that have the GPU to themselves: the
+    // launch's work-groups wait for each other, and two of them at once could
+    // each hold CUs the other waits for.  Set by the single-replica ABI; the
+    // replica engine runs the sweeps (the same bits).  Cleared when a solve was
+    // abandoned (another process waits on the same GPU).
+    int onchip = 0;
+    CgOnchip onchip_w{nullptr, nullptr, 1u};
+    int onchip_void = 0;           // tests: the next launch starts abandoned
+    unsigned int onchip_span = 0;  // epochs the last such solve may have used
+    // Whether the next solve on grid d goes on the chip (sets its exchange up).
+    bool onchip_next(const GridDims& d, int limit, int two = 0);
+    // FP64 CG runs with one reduction per iteration (Cg1) in the FP64 precisions.
+    // The mixed ones' cold solves keep two: an FP32 inner solve turns a last-bit
+    // difference of its start into 2.6e-9 of the forces after 200 steps (4096
+    // ions / 128^3), so those trajectories stay, bit for bit, what they were.
+    bool cg_two() const { return precision == kMixedCG || precision == kMixedMG; }
+    CgRun cg_run(double* x, const double* b, int chunk, int* pred) const {
+        return CgRun{cg_two() ? dims : cgd, pbc(), x, r, p0, p1, n * n, 0, chunk, pred, b, tol,
+                     cg_two() ? 1 : 0, 0};
+    }
     // A mixed-precision solve in progress (mixed_issue .. mixed_finish).
     struct MixedRun {
         bool use_mg = false, extrap = false;
@@ -344,8 +366,7 @@ struct Sim {
     void momentum(double* out);
 
     // solvers
-    int cg_solve(const GridDims& d, const PBCoef& pbc, const double* b, double* x, double tol,
-                 int limit, double* rbuf, double* pa, double* pbuf, int* pred);
+    int cg_solve(const CgRun& c);
     int cg_count_solve(const GridDims& d, const PBCoef& cpb, const double* b, double* x,
                        double rtol, int maxit, double* rbuf, double* pa, double* pbuf, int* pred,
                        CGState* cst);
@@ -412,7 +433,8 @@ struct Sim {
     int mixed_finish();
     void mixed_refine(int add);
     void mixed_pass(int k, int m, bool poll);
-    void cg_issue(const CgRun& c, const double* b, double tol);
+    void cg_issue(const CgRun& c);
+    void cg_start();
     void cg_chunk();
     int cg_finish();
     int lcg_update();

@@ -289,6 +289,91 @@ struct BodyUpdate {
     }
 };
 
+// ---- CG with one reduction per iteration ---------------------------------------
+// The iteration of library/src/plcg.c:28-90 needs <p, A p> before the update
+// and <r, r> after it.  Its second sum follows from sums over the same pass as
+// the first, since r' = r + alpha A p:
+//   <r', r'> = <r, r> + 2 alpha <r, A p> + alpha^2 <A p, A p>
+// (G. Meurant, Multitasking the conjugate gradient method on the CRAY X-MP/48,
+// Parallel Computing 5 (1987) 267).  Only beta is formed from it: the next pass
+// sums <r', r'> itself, which alpha and the stop test use, so its rounding does
+// not build up.
+__device__ __forceinline__ void cg1_terms(double p, double r, double lap, double (&s)[kCg1Sums],
+                                          double& m) {
+    s[0] += p * lap;
+    s[1] += r * lap;
+    s[2] += lap * lap;
+    s[3] += r * r;
+    m = fmax(m, fabs(r));
+}
+
+// The four wave results of a tile in order, and a pair of tiles'.
+__device__ __forceinline__ double cg1_tile(const double* w) { return ((w[0] + w[1]) + w[2]) + w[3]; }
+__device__ __forceinline__ double cg1_pair(const double* a, const double* b) {
+    return cg1_tile(a) + cg1_tile(b);
+}
+__device__ __forceinline__ double cg1_pair_max(const double* a, const double* b) {
+    return fmax(fmax(fmax(a[0], a[1]), fmax(a[2], a[3])), fmax(fmax(b[0], b[1]), fmax(b[2], b[3])));
+}
+
+// 64 partials of 5 values (the sums and the max): lane 8 j + c holds value c of
+// partials j, j + 8, ..., j + 56 in v and adds them in this order, then the
+// eight lanes of a value by halves.  maxi: this lane's value is the max.
+// All lanes get their value's result.
+__device__ __forceinline__ double cg1_fold(const double (&v)[8], bool maxi) {
+    double t = v[0];
+#pragma unroll
+    for (int i = 1; i < 8; i++) t = maxi ? fmax(t, v[i]) : t + v[i];
+    double o = dpp_move<kDppRor8>(t);
+    t = maxi ? fmax(t, o) : t + o;
+    o = __shfl_xor(t, 16);
+    t = maxi ? fmax(t, o) : t + o;
+    o = __shfl_xor(t, 32);
+    return maxi ? fmax(t, o) : t + o;
+}
+
+struct Cg1 {
+    double rdv = 0.0, pAp = 0.0, alpha = 0.0, beta = 0.0, rr = 0.0, rmax = 0.0;
+    // S: the sums of cg1_terms, M: max|r| before the update of iteration `iter`
+    // (0-based).  True: the solve stops there, with `res` as BodyUpdate::finalize
+    // gives it.
+    __device__ __forceinline__ bool decide(const double* S, double M, int iter, int limit,
+                                           int count_mode, int plain, double tol, double stop,
+                                           int& res) {
+        rr = S[3];
+        rmax = M;
+        if (iter > 0) {
+            if (M <= (count_mode ? stop : tol)) {
+                res = count_mode ? iter : iter - 1;
+                return true;
+            }
+            if (iter >= limit) {
+                res = count_mode ? limit : -1;
+                return true;
+            }
+        }
+        pAp = S[0];
+        if (fabs(pAp) < 1e-300) {  // breakdown guard, as BodyDir
+            alpha = 0.0;
+            res = iter;
+            return true;
+        }
+        rdv = plain ? rr : -rr / 6.0;
+        alpha = rdv / pAp;
+        beta = fmax(rr + alpha * (2.0 * S[1] + alpha * S[2]), 0.0) / rr;
+        return false;
+    }
+    __device__ __forceinline__ void store(CGState* st) const {
+        st->rdv = rdv;
+        st->pAp = pAp;
+        st->alpha = alpha;
+        st->beta = beta;
+        st->rr = rr;
+        st->rmax = rmax;
+        st->first = 0;
+    }
+};
+
 // ---- deferred finalisation ----------------------------------------------------
 // The producer writes one partial per work-group with a plain store and ends;
 // every work-group of the consumer folds all partials itself, in the same

@@ -1,0 +1,100 @@
+"""The one-launch CG (vectors on the chip) against the sweeps, bit for bit."""
+import ctypes
+
+import numpy as np
+import pytest
+
+D = np.ctypeslib.ndpointer(dtype=np.float64, flags="C_CONTIGUOUS")
+FIT_MAX = 128  # the largest grid whose vectors fit
+
+
+def _solve(hip_raw, b, x, tol, n, reductions, onchip, coef=None):
+    f = hip_raw.maze_test_conj_grad_form
+    P = ctypes.c_void_p
+    f.restype = ctypes.c_int
+    f.argtypes = [D, D, ctypes.c_double, ctypes.c_int, P, P, P, P, ctypes.c_int, ctypes.c_int]
+    ptrs = [None] * 4 if coef is None else [c.ctypes.data for c in coef]
+    return f(b, x, tol, n, *ptrs, reductions, onchip)
+
+
+def _problem(n, seed):
+    g = np.random.default_rng(seed)
+    b = g.normal(size=(n, n, n))
+    return b - b.mean(), g.normal(size=(n, n, n)) * 1e-3
+
+
+# Slab heights 1 to 16, one to four tiles per work-group, partly filled last
+# tiles and slabs, windows that wrap onto themselves.
+@pytest.mark.gpu
+@pytest.mark.parametrize("reductions", [1, 2])
+@pytest.mark.parametrize("n", [2, 5, 16, 23, 31, 32, 48, 57, 64, 73, 81, 100, 113, 126, 127,
+                               FIT_MAX])
+def test_onchip_cg_equals_sweeps(hip_raw, n, reductions):
+    b, x0 = _problem(n, n)
+    tol = 1e-7 * np.abs(b).max()
+    xs, xo = x0.copy(), x0.copy()
+    i_s = _solve(hip_raw, b, xs, tol, n, reductions, 0)
+    i_o = _solve(hip_raw, b, xo, tol, n, reductions, 1)
+    assert i_o == i_s and i_s >= 0
+    assert np.array_equal(xo, xs)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("reductions", [1, 2])
+@pytest.mark.parametrize("n", [16, 48, 73, 100, FIT_MAX])
+def test_onchip_pb_cg_equals_sweeps(hip_raw, n, reductions):
+    b, x0 = _problem(n, n)
+    g = np.random.default_rng(7)
+    coef = [g.uniform(2.0, 80.0, (n, n, n)) for _ in range(3)] + [g.uniform(0.0, 0.1, (n, n, n))]
+    tol = 1e-7 * np.abs(b).max()
+    xs, xo = x0.copy(), x0.copy()
+    i_s = _solve(hip_raw, b, xs, tol, n, reductions, 0, coef)
+    i_o = _solve(hip_raw, b, xo, tol, n, reductions, 1, coef)
+    assert i_o == i_s and i_s >= 0
+    assert np.array_equal(xo, xs)
+
+
+# The one-reduction recurrence against the two-reduction one: the same iterates up to
+# rounding.  A relative difference of 1e-16 per sum stays within 1e-10 of the solution
+# over a solve of under 300 iterations.
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [16, 48, 81, FIT_MAX])
+def test_one_reduction_equals_two(hip_raw, n):
+    b, x0 = _problem(n, n)
+    tol = 1e-6 * np.abs(b).max()
+    x1, x2 = x0.copy(), x0.copy()
+    i1 = _solve(hip_raw, b, x1, tol, n, 1, 0)
+    i2 = _solve(hip_raw, b, x2, tol, n, 2, 0)
+    assert i1 == i2
+    assert np.linalg.norm(x1 - x2) <= 1e-10 * np.linalg.norm(x2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("reductions", [1, 2])
+def test_onchip_cg_limits(hip_raw, reductions):
+    n = FIT_MAX + 2
+    b, x = _problem(n, 1)
+    assert _solve(hip_raw, b, x, 1.0, n, reductions, 1) == -2
+    # A zero residual stops before the first direction, with x unchanged.
+    n = 20
+    z, x = np.zeros((n, n, n)), np.full((n, n, n), 3.0)
+    assert _solve(hip_raw, z, x, 1e-9, n, reductions, 1) == 0 and (x == 3.0).all()
+    # An unreachable tolerance ends at the iteration cap n^2.
+    n = 6
+    b, x = _problem(n, 2)
+    xs = x.copy()
+    assert _solve(hip_raw, b, xs, 0.0, n, reductions, 0) == _solve(hip_raw, b, x, 0.0, n, reductions, 1)
+    assert np.array_equal(x, xs)
+
+
+# A launch that finds its solve abandoned leaves x alone, and the sweeps run it.
+@pytest.mark.gpu
+@pytest.mark.parametrize("reductions", [1, 2])
+def test_abandoned_launch_falls_back(hip_raw, reductions):
+    n = 64
+    b, x0 = _problem(n, 3)
+    tol = 1e-6 * np.abs(b).max()
+    xs, xo = x0.copy(), x0.copy()
+    assert _solve(hip_raw, b, xs, tol, n, reductions, 0) >= 0
+    assert _solve(hip_raw, b, xo, tol, n, reductions, 2) == -3
+    assert np.array_equal(xo, xs)
