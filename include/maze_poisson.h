@@ -193,7 +193,10 @@ void get_eps_k2(double *eps_x, double *eps_y, double *eps_z, double *k2);
 /* Field-solve arithmetic: 0 = FP64 CG as in the reference (default);
  * 1 = FP32-storage CG inside FP64 iterative refinement, stopping on the
  * reference's criterion max|A y - sigma| <= tol evaluated in FP64;
- * 2 = as 1 with the multigrid-preconditioned FP32 CG below;
+ * 2 = as 1 with the multigrid-preconditioned FP32 CG below, or, at tolerances
+ * below 1e-9 of 4 pi max|q| / (h eps) on an even grid of at most 256^3 (Poisson
+ * operator, default inner stop, no extrapolation), a direct FP64 solve, held to
+ * the same stop test;
  * 3 = FP64 CG preconditioned by mode 2's V-cycle carried out in FP64, to the
  * same stop test (MAZE-LCG on the Poisson operator where mode 2 runs the
  * one-work-group coarsest solve; otherwise the MaZe solve runs mode 0).
@@ -276,6 +279,9 @@ int maze_test_conj_grad_pb(const double *b, double *x, double tol, int n, const 
 int maze_test_conj_grad_form(const double *b, double *x, double tol, int n, const double *eps_x,
                              const double *eps_y, const double *eps_z, const double *k2,
                              int reductions, int onchip);
+/* The direct Poisson solve (n even, at most 256; x without the constant mode);
+ * returns n, or -1 for another n. */
+int maze_test_spectral(const double *b, double *x, int n);
 void maze_test_rbgs(const double *in, double *out, int n, int iters);
 int maze_test_restrict27(const double *in, double *out, int n);
 int maze_test_prolong_add(const double *in, double *out, int nc);

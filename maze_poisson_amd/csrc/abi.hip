@@ -411,6 +411,17 @@ int maze_test_conj_grad_pb(const double* b, double* x, double tol, int n, const 
     return maze_test_conj_grad_form(b, x, tol, n, ex, ey, ez, k2, 1, 0);
 }
 
+int maze_test_spectral(const double* b, double* x, int n) {
+    if (!maze::spectral_ok(n)) return -1;
+    Sim* s = scratch_sim(n);
+    MAZE_HIP(hipMemcpy(s->sigma, b, s->G * sizeof(double), hipMemcpyHostToDevice));
+    s->direct_solve(s->sigma, s->y);
+    s->sync();
+    MAZE_HIP(hipMemcpy(x, s->y, s->G * sizeof(double), hipMemcpyDeviceToHost));
+    delete s;
+    return n;
+}
+
 void maze_test_rbgs(const double* in, double* out, int n, int iters) {
     Sim* s = scratch_sim(n);
     MAZE_HIP(hipMemcpy(s->sigma, in, s->G * sizeof(double), hipMemcpyHostToDevice));

@@ -121,6 +121,7 @@ static long long arena_bytes(int n, int np, int precision, const Phys& ph) {
         b += 8 * G + 8 * kBlockJacobiTab;             // preconditioned residual, eigenbasis tables
     if (ph.pb) b += 4 * 8 * G;                        // dielectric maps and screening
     if (precision != kFP64) b += 8 * G + 4 * 4 * G;   // second y, FP32 d, r, p0, p1
+    if (precision == kMixedMG && !ph.pb && spectral_ok(n)) b += 8LL * spectral_doubles(n);
     if (precision == kMixedMG) {
         const std::vector<int> sz = Sim::mg_sizes(n);
         for (size_t l = 0; l < sz.size(); l++) {

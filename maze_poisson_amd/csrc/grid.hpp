@@ -151,6 +151,16 @@ long cg_onchip_words();
 void launch_cg_onchip(hipStream_t s, const GridDims& d, const PBCoef& pb, double* x, double* r,
                       double* h0, double* h1, CGState* st, const CgOnchip& w);
 
+// Direct FP64 solve A x = b (Poisson operator, without the constant mode) by
+// the transform of each axis, n even and at most 256 (spectral.hip).  tab:
+// spectral_doubles(n) values of spectral_tables in device memory; w: a scratch
+// grid; b, x and w do not overlap.
+bool spectral_ok(int n);
+long spectral_doubles(int n);
+void spectral_tables(int n, double* tab);
+void launch_spectral_solve(hipStream_t s, int n, const double* tab, const double* b, double* x,
+                           double* w);
+
 // Mixed precision, FP64 true residual of the refinement loop, b = sigma - A y.
 // First pass (add_d == 0): y = y0, starts the loop (ysel = 0).
 // Later passes: y_new = y + d with y/y_new the two buffers y0/y1 selected by

@@ -187,6 +187,7 @@ void Sim::free_grid() {
                        &mg_r, &c_rhs, &c_eps, &c_r, &c_p0, &c_p1, &pv, &bj_tab})
         dfree(*a);
     for (float** a : {&d32, &r32, &q32a, &q32b}) dfree(*a);
+    dfree(spec_tab);
     for (double** a : {&cex, &cey, &cez, &ck2}) dfree(*a);
     free_mg();
     free_pbmg();
@@ -313,6 +314,9 @@ void Sim::init_particles(int n_, int n_typ, double L_, double h_, int np, int ca
     p.cas = cas;
     p.nn = cas == 0 ? 8 : 64;
     p.r_cut = L_ / 2.0;
+    qmax = 0.0;
+    for (int i = 0; i < np; i++) qmax = std::max(qmax, std::fabs(charges[i]));
+    if (!(qmax > 0.0)) qmax = 1.0;
     p.types = dalloc<int>(np);
     p.pos = dalloc<double>(3L * np); p.vel = dalloc<double>(3L * np);
     p.mass = dalloc<double>(np); p.charges = dalloc<double>(np);
@@ -1225,6 +1229,13 @@ void Sim::mixed_issue() {
     m.ya = m.extrap ? y_alt : y;
     m.yb = m.extrap ? y_hist : y_alt;
     if (y_extrap && !hist_ok) launch_copy(stream, G, y, y_hist);
+    // A direct solve meets the stop test in the first refinement pass, which
+    // applies it; should rounding keep it above the tolerance, the loop goes on
+    // from there.
+    if (use_direct()) {
+        sched.clear();
+        direct_solve(sigma, y);
+    }
     if (m.extrap)
         timed(kTRefine, 0, [&] {
             launch_refine_extrap(stream, dims, pbc(), y, y_hist, y_alt, sigma, r32, m.ra, st, red);
@@ -1236,6 +1247,17 @@ void Sim::mixed_issue() {
         mixed_pass(m.queued, k >= 0 ? std::max(k, 1) : 1 - k, false);
     }
     publish();
+}
+
+void Sim::direct_solve(const double* b, double* x) {
+    if (!spec_tab) {
+        const long k = spectral_doubles(n);
+        std::vector<double> tab(k);
+        spectral_tables(n, tab.data());
+        spec_tab = dalloc<double>(k);
+        MAZE_HIP(hipMemcpy(spec_tab, tab.data(), k * sizeof(double), hipMemcpyHostToDevice));
+    }
+    launch_spectral_solve(stream, n, spec_tab, b, x, r);
 }
 
 // Each refinement pass also starts the next pass's inner solve.
@@ -1543,8 +1565,10 @@ void Sim::cold_issue() {
     m.extrap = false;
     m.ya = phi;
     m.yb = tmp;
+    const bool direct = use_direct();
+    if (direct) direct_solve(sigma, phi);
     mixed_refine(0);
-    for (m.queued = 0; m.queued < kColdPasses; m.queued++)
+    for (m.queued = 0; m.queued < (direct ? 0 : kColdPasses); m.queued++)
         mixed_pass(m.queued, std::min(kColdIters, m.inner_limit), false);
     publish();
 }
