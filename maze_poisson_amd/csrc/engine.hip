@@ -45,6 +45,12 @@ double quantile(std::vector<double> v, double q) {
 
 }  // namespace
 
+// What a running replica borrows from the engine.
+struct Lane {
+    hipStream_t main = nullptr, side = nullptr;
+    HostBlock* host = nullptr;
+};
+
 // Physics of a request beyond maze_engine_submit's defaults (MAZE-LCG without
 // a preconditioner, CIC, Tosi-Fumi, velocity Verlet without thermostat).
 struct Phys {
@@ -80,7 +86,7 @@ struct Request {
     double t_admit = 0, t_done = 0, t_last = 0;
     std::vector<double> lat;  // seconds per step, as observed by the loop
     std::unique_ptr<Sim> sim;
-    std::pair<hipStream_t, hipStream_t> streams{nullptr, nullptr};
+    Lane lane;
     std::vector<double> out_pos, out_vel, out_f, out_phi;
     double obs[7] = {0, 0, 0, 0, 0, 0, 0};  // kinetic, temperature, E_elec, V_TF, momentum
 };
@@ -197,9 +203,10 @@ struct Engine {
     double host_admit = 0, host_issue = 0, host_finish = 0;  // host seconds per phase
     int run_threads = 1;  // worker threads of the current run
 
-    // Streams of retired replicas, reused by the next ones (creating a stream
-    // costs milliseconds); destroyed with the engine.
-    std::vector<std::pair<hipStream_t, hipStream_t>> stream_pool;
+    // Streams and pinned blocks of retired replicas, reused by the next ones
+    // (creating a stream costs milliseconds, freeing a pinned block 0.2 ms);
+    // destroyed with the engine.
+    std::vector<Lane> lane_pool;
 
     // New streams come Q main streams, then their Q side streams, Q being the
     // runtime's hardware queues per process (GPU_MAX_HW_QUEUES, four by
@@ -210,34 +217,36 @@ struct Engine {
     // `created` gets the drop of free device memory over a new batch: the
     // runtime sets up its hardware queues (a per-process cost, at most four
     // queues) as the first streams are made, so it is not a per-replica cost.
-    std::pair<hipStream_t, hipStream_t> take_streams(long long& created) {
+    Lane take_lane(long long& created) {
         created = 0;
         std::lock_guard<std::mutex> g(mu);
-        if (stream_pool.empty()) {
+        if (lane_pool.empty()) {
             const int q = hw_queues();
             size_t f0 = 0, f1 = 0, total = 0;
             MAZE_HIP(hipMemGetInfo(&f0, &total));
             std::vector<hipStream_t> mains(q), sides(q);
             for (auto& m : mains) MAZE_HIP(hipStreamCreateWithFlags(&m, hipStreamNonBlocking));
             for (auto& sd : sides) MAZE_HIP(hipStreamCreateWithFlags(&sd, hipStreamNonBlocking));
-            for (int k = q - 1; k >= 0; k--) stream_pool.push_back({mains[k], sides[k]});
+            for (int k = q - 1; k >= 0; k--)
+                lane_pool.push_back({mains[k], sides[k], host_block_create()});
             MAZE_HIP(hipMemGetInfo(&f1, &total));
             created = (long long)f0 - (long long)f1;
         }
-        auto p = stream_pool.back();
-        stream_pool.pop_back();
-        return p;
+        const Lane l = lane_pool.back();
+        lane_pool.pop_back();
+        return l;
     }
 
-    void give_streams(std::pair<hipStream_t, hipStream_t> p) {
+    void give_lane(const Lane& l) {
         std::lock_guard<std::mutex> g(mu);
-        stream_pool.push_back(p);
+        lane_pool.push_back(l);
     }
 
     ~Engine() {
-        for (auto& p : stream_pool) {
-            MAZE_HIP(hipStreamDestroy(p.first));
-            MAZE_HIP(hipStreamDestroy(p.second));
+        for (Lane& l : lane_pool) {
+            MAZE_HIP(hipStreamDestroy(l.main));
+            MAZE_HIP(hipStreamDestroy(l.side));
+            host_block_destroy(l.host);
         }
     }
 
@@ -245,16 +254,18 @@ struct Engine {
     // start-up steps with cold solves and the first step's issue.
     void admit(Request& r) {
         r.used_precision = precision_for(r.n, r.precision, r.ph);
-        // Streams come from the pool, created four pairs at a time and counted
-        // apart from the replica's own memory.
-        r.streams = take_streams(r.stream_bytes);
+        // Its lane comes from the pool, created four at a time and counted apart
+        // from the replica's own memory.
+        r.lane = take_lane(r.stream_bytes);
         size_t free0 = 0, total = 0;
         MAZE_HIP(hipMemGetInfo(&free0, &total));
         r.arena = std::make_unique<DevArena>();
         r.arena->size = (size_t)arena_bytes(r.n, r.np, r.used_precision, r.ph);
         MAZE_HIP(hipMalloc(&r.arena->base, r.arena->size));
+        MAZE_HIP(hipMemsetAsync(r.arena->base, 0, r.arena->size, r.lane.main));
+        MAZE_HIP(hipStreamSynchronize(r.lane.main));
         arena_install(r.arena.get());
-        r.sim = std::make_unique<Sim>(r.streams.first, r.streams.second);
+        r.sim = std::make_unique<Sim>(r.lane.main, r.lane.side, r.lane.host);
         Sim& s = *r.sim;
         const double h = r.L / r.n;
         const Phys& ph = r.ph;
@@ -354,8 +365,7 @@ struct Engine {
                                hipMemcpyDeviceToHost));
         }
         r.sim.reset();  // waits for both streams
-        give_streams(r.streams);
-        arena_forget(r.arena.get());
+        give_lane(r.lane);
         MAZE_HIP(hipFree(r.arena->base));
         r.arena.reset();
         r.state = 2;

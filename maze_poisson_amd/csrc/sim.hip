@@ -28,57 +28,66 @@ static void fatal(const char* msg) {
 }
 
 // Device arenas: while one is installed on the calling thread, replica
-// allocations are carved from it (256-byte aligned) instead of hipMalloc;
-// allocations that do not fit fall back to hipMalloc and are counted.
+// allocations are carved from it (256-byte aligned) instead of the replica's own
+// chunks; allocations that do not fit fall back to a chunk and are counted.
 namespace {
 thread_local DevArena* t_arena = nullptr;
-std::mutex g_arena_mu;
-std::vector<const DevArena*> g_arenas;  // live arenas, for dfree
-
-bool in_arena(const void* p) {
-    const char* c = static_cast<const char*>(p);
-    std::lock_guard<std::mutex> g(g_arena_mu);
-    for (const DevArena* a : g_arenas)
-        if (c >= a->base && c < a->base + a->size) return true;
-    return false;
-}
 }  // namespace
 
-void arena_install(DevArena* a) {
-    t_arena = a;
-    std::lock_guard<std::mutex> g(g_arena_mu);
-    if (a && std::find(g_arenas.begin(), g_arenas.end(), a) == g_arenas.end()) g_arenas.push_back(a);
-}
+void arena_install(DevArena* a) { t_arena = a; }
 
-void arena_forget(const DevArena* a) {
-    if (t_arena == a) t_arena = nullptr;
-    std::lock_guard<std::mutex> g(g_arena_mu);
-    g_arenas.erase(std::remove(g_arenas.begin(), g_arenas.end(), a), g_arenas.end());
-}
-
-template <class T>
-static T* dalloc(long count) {
-    T* p = nullptr;
-    if (count <= 0) count = 1;
-    const size_t bytes = sizeof(T) * (size_t)count;
-    if (DevArena* a = t_arena) {
-        const size_t off = (a->used + kArenaAlign - 1) & ~(kArenaAlign - 1);
-        if (off + bytes <= a->size) {
-            p = reinterpret_cast<T*>(a->base + off);
-            a->used = off + bytes;
-        } else {
-            a->overflow += bytes;
+// A replica's device memory comes in a few zeroed chunks (reserve()), carved like
+// an arena; a chunk is freed with its last allocation.  A hipMalloc, hipMemset
+// and hipFree for each of some 60 arrays took 5 ms of a 4096-ion / 128^3
+// replica's life, 0.9 ms of it the clearing and 3.6 ms the freeing.
+char* Sim::carve(size_t bytes) {
+    bytes = (bytes + kArenaAlign - 1) & ~(kArenaAlign - 1);
+    if (DevArena* a = t_arena) {  // cleared by its owner
+        if (a->used + bytes <= a->size) {
+            char* p = a->base + a->used;
+            a->used += bytes;
+            return p;
         }
+        a->overflow += bytes;
     }
-    if (!p) MAZE_HIP(hipMalloc(&p, bytes));
-    MAZE_HIP(hipMemset(p, 0, bytes));
+    auto room = [&](const Chunk& c) { return c.used + bytes <= c.size; };
+    auto it = std::find_if(chunks.rbegin(), chunks.rend(), room);
+    if (it == chunks.rend()) {
+        add_chunk(std::max(bytes, kMinChunk));
+        it = chunks.rbegin();
+    }
+    char* p = it->base + it->used;
+    it->used += bytes;
+    it->live++;
     return p;
 }
 
-template <class T>
-static void dfree(T*& p) {
-    if (p && !in_arena(p)) MAZE_HIP(hipFree(p));
-    p = nullptr;
+void Sim::add_chunk(size_t bytes) {
+    Chunk c;
+    c.size = bytes;
+    MAZE_HIP(hipMalloc(&c.base, bytes));
+    MAZE_HIP(hipMemsetAsync(c.base, 0, bytes, stream));
+    MAZE_HIP(hipStreamSynchronize(stream));
+    chunks.push_back(c);
+}
+
+// One chunk for allocations of `bytes` in all, about to be made in `count` calls.
+void Sim::reserve(size_t bytes, int count) {
+    if (!t_arena) add_chunk(bytes + (size_t)count * kArenaAlign);
+}
+
+// Returns an allocation to its chunk (an arena's is its owner's to free).
+void Sim::uncarve(void* p) {
+    char* q = static_cast<char*>(p);
+    for (size_t i = 0; i < chunks.size(); i++) {
+        Chunk& c = chunks[i];
+        if (q < c.base || q >= c.base + c.size) continue;
+        if (--c.live == 0) {
+            MAZE_HIP(hipFree(c.base));
+            chunks.erase(chunks.begin() + (long)i);
+        }
+        return;
+    }
 }
 
 // Planes per work-group so that one sweep launches about 512 work-groups.
@@ -101,11 +110,20 @@ static int choose_slab(int n) {
 
 GridDims grid_dims_for(int n) { return make_dims(n, choose_slab(n)); }
 
-Sim::Sim() : Sim(nullptr, nullptr) {}
+Sim::Sim() : Sim(nullptr, nullptr, nullptr) {}
 
-// main / side: streams the caller keeps (both or neither), for callers that
-// create many replicas (stream creation costs milliseconds).
-Sim::Sim(hipStream_t main, hipStream_t side_) {
+HostBlock* host_block_create() {
+    HostBlock* b = nullptr;
+    MAZE_HIP(hipHostMalloc(&b, sizeof(HostBlock), hipHostMallocCoherent | hipHostMallocMapped));
+    return b;
+}
+
+void host_block_destroy(HostBlock* b) { MAZE_HIP(hipHostFree(b)); }
+
+// main / side / block: streams and pinned memory the caller keeps (all or none),
+// for callers that create many replicas (creating streams costs milliseconds,
+// freeing pinned memory 0.2 ms).
+Sim::Sim(hipStream_t main, hipStream_t side_, HostBlock* block) {
     own_streams = main == nullptr;
     if (own_streams) {
         MAZE_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
@@ -116,6 +134,14 @@ Sim::Sim(hipStream_t main, hipStream_t side_) {
     }
     MAZE_HIP(hipEventCreateWithFlags(&ev_pos, hipEventDisableTiming));
     MAZE_HIP(hipEventCreateWithFlags(&ev_tf, hipEventDisableTiming));
+    host = own_streams ? host_block_create() : block;
+    std::memset(static_cast<void*>(host), 0, sizeof(HostBlock));
+    st_host = &host->st;
+    hscalar = host->scalars;
+    ps_host = &host->ps;
+    pub_host = &host->pub;
+    MAZE_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&pub_dev), pub_host, 0));
+    reserve(sizeof(double) * (7 + kCg1Sums) * (size_t)kMaxPartials + (64 << 10), 16);
     red_side.psum = dalloc<double>(kMaxPartials);
     red_side.pmax = dalloc<double>(kMaxPartials);
     red_side.counter = dalloc<unsigned int>(kArrivalWords);
@@ -127,8 +153,6 @@ Sim::Sim(hipStream_t main, hipStream_t side_) {
     if (const char* e = std::getenv("MAZE_MG_FUSE_COARSE")) mg_fuse_coarse = std::atoi(e) != 0;
     st = dalloc<CGState>(1);
     st_c = dalloc<CGState>(1);
-    MAZE_HIP(hipHostMalloc(&st_host, sizeof(CGState)));
-    std::memset(st_host, 0, sizeof(CGState));
     red.psum = dalloc<double>((long)kCg1Sums * kMaxPartials);
     red.pmax = dalloc<double>(kMaxPartials);
     red.counter = dalloc<unsigned int>(kArrivalWords);
@@ -137,12 +161,7 @@ Sim::Sim(hipStream_t main, hipStream_t side_) {
     dred.pus = dalloc<double>(kMaxPartials);
     dred.pum = dalloc<double>(kMaxPartials);
     dscalar = dalloc<double>(8);
-    MAZE_HIP(hipHostMalloc(&hscalar, 8 * sizeof(double)));
     ps = dalloc<PScalars>(1);
-    MAZE_HIP(hipHostMalloc(&ps_host, sizeof(PScalars)));
-    MAZE_HIP(hipHostMalloc(&pub_host, sizeof(StatePub), hipHostMallocCoherent | hipHostMallocMapped));
-    std::memset(pub_host, 0, sizeof(StatePub));
-    MAZE_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&pub_dev), pub_host, 0));
 }
 
 Sim::~Sim() {
@@ -169,10 +188,8 @@ Sim::~Sim() {
     dfree(ps);
     dfree(onchip_w.words);
     dfree(onchip_w.ctl);
-    if (st_host) MAZE_HIP(hipHostFree(st_host));
-    if (hscalar) MAZE_HIP(hipHostFree(hscalar));
-    if (ps_host) MAZE_HIP(hipHostFree(ps_host));
-    if (pub_host) MAZE_HIP(hipHostFree(pub_host));
+    for (Chunk& c : chunks) MAZE_HIP(hipFree(c.base));
+    if (own_streams) host_block_destroy(host);
     for (auto e : ev_pool) MAZE_HIP(hipEventDestroy(e));
     MAZE_HIP(hipEventDestroy(ev_pos));
     MAZE_HIP(hipEventDestroy(ev_tf));
@@ -252,11 +269,14 @@ void Sim::init_grid(int n_, double L_, double h_, double tol_, double eps, doubl
     dims = grid_dims_for(n);
     cgd = cg_dims_for(n);
     if (dims.blocks > kMaxPartials) fatal("maze: grid too large for the reduction buffers");
+    const bool two_grid = type == kMG || type == kMazeMG || (type == kMazeLCG && precond_ == kPMG);
+    reserve(sizeof(double) * (size_t)G * (9 + (two_grid ? 3 : 0) +
+                                          (precond_ == kPBlockJacobi ? 1 : 0)) + (64 << 10), 24);
     q = dalloc<double>(G); y = dalloc<double>(G); phi = dalloc<double>(G);
     spread_zero_old = 0;
     phip = dalloc<double>(G); tmp = dalloc<double>(G); sigma = dalloc<double>(G);
     r = dalloc<double>(G); p0 = dalloc<double>(G); p1 = dalloc<double>(G);
-    if (type == kMG || type == kMazeMG || (type == kMazeLCG && precond_ == kPMG)) {
+    if (two_grid) {
         nc = n / 2;
         cdims = cg_dims_for(nc);
         const long Gc = (long)nc * nc * nc;
@@ -281,6 +301,7 @@ void Sim::init_grid(int n_, double L_, double h_, double tol_, double eps, doubl
 void Sim::init_pb(double w_, double kbar2_, int nonpolar_) {
     pb = 1; w = w_; kbar2 = kbar2_; nonpolar = nonpolar_;
     pbmg_dirty = 1;
+    reserve(4 * sizeof(double) * (size_t)G, 4);
     ex = dalloc<double>(G); ey = dalloc<double>(G); ez = dalloc<double>(G); k2 = dalloc<double>(G);
     launch_fill(stream, G, 1.0, ex);
     launch_fill(stream, G, 1.0, ey);
@@ -317,6 +338,8 @@ void Sim::init_particles(int n_, int n_typ, double L_, double h_, int np, int ca
     qmax = 0.0;
     for (int i = 0; i < np; i++) qmax = std::max(qmax, std::fabs(charges[i]));
     if (!(qmax > 0.0)) qmax = 1.0;
+    reserve((size_t)np * (4 + 5 * 24 + 2 * 8 + 12 + 4 + p.nn * (8 + 4 + 4) + 8) +
+                8 * ((size_t)n_ * n_ * n_ + tf_part_doubles(np) + 7L * n_typ * n_typ), 20);
     p.types = dalloc<int>(np);
     p.pos = dalloc<double>(3L * np); p.vel = dalloc<double>(3L * np);
     p.mass = dalloc<double>(np); p.charges = dalloc<double>(np);
@@ -1200,13 +1223,21 @@ int Sim::maze_mixed() {
     return mixed_finish();
 }
 
+// The arrays of the mixed path (and, for its levels, room for a hierarchy: two
+// more FP32 arrays on the finest level, three on those below, or the PB levels'
+// seven and eight).
+void Sim::mixed_arrays() {
+    if (d32) return;
+    const size_t levels = precision != kMixedMG ? 0 : pb ? 7 + 2 : 2 + 1;
+    reserve((size_t)G * (8 + 4 * 4 + 4 * levels), 5);
+    d32 = dalloc<float>(G); r32 = dalloc<float>(G);
+    q32a = dalloc<float>(G); q32b = dalloc<float>(G); y_alt = dalloc<double>(G);
+}
+
 // Everything up to the publication of the state after the previous step's
 // schedule of passes.
 void Sim::mixed_issue() {
-    if (!d32) {
-        d32 = dalloc<float>(G); r32 = dalloc<float>(G);
-        q32a = dalloc<float>(G); q32b = dalloc<float>(G); y_alt = dalloc<double>(G);
-    }
+    mixed_arrays();
     if (y_extrap && !y_hist) y_hist = dalloc<double>(G);
     MixedRun& m = mx;
     m.use_mg = precision == kMixedMG && (pb ? setup_pbmg() : setup_mg());
@@ -1549,10 +1580,7 @@ void Sim::init_field_finish() {
 // met its tolerance, and passes after the loop has, are no-ops); further
 // passes are polled.  The MD steps' pass schedule is left alone.
 void Sim::cold_issue() {
-    if (!d32) {
-        d32 = dalloc<float>(G); r32 = dalloc<float>(G);
-        q32a = dalloc<float>(G); q32b = dalloc<float>(G); y_alt = dalloc<double>(G);
-    }
+    mixed_arrays();
     MixedRun& m = mx;
     m.use_mg = precision == kMixedMG && (pb ? setup_pbmg() : setup_mg());
     if (m.use_mg && !pb) mg[0].b = r32;

@@ -18,18 +18,27 @@ enum ItgType { kOVRVO = 0, kVerlet = 1 };
 // (the same solver without the FP32 storage; Poisson operator only).
 enum Precision { kFP64 = 0, kMixedCG = 1, kMixedMG = 2, kFP64MG = 3 };
 
-// A block of device memory that replica allocations are carved from while it
-// is installed (arena_install) on the allocating thread: one hipMalloc per
+// A block of zeroed device memory that replica allocations are carved from while
+// it is installed (arena_install) on the allocating thread: one hipMalloc per
 // replica and an exact account of its footprint.  dfree leaves arena memory
-// alone; the owner frees the block after arena_forget.
+// alone; the owner frees the block once the replica is gone.
 constexpr size_t kArenaAlign = 256;
 struct DevArena {
     char* base = nullptr;
     size_t size = 0, used = 0;
     size_t overflow = 0;  // bytes that did not fit and came from hipMalloc
 };
-void arena_install(DevArena* a);  // nullptr: plain hipMalloc again
-void arena_forget(const DevArena* a);
+void arena_install(DevArena* a);  // nullptr: the replica's own chunks again
+
+// What a replica exchanges with the host, in one pinned, host-coherent block.
+struct HostBlock {
+    StatePub pub;
+    CGState st;
+    PScalars ps;
+    double scalars[8];
+};
+HostBlock* host_block_create();
+void host_block_destroy(HostBlock* b);
 
 // One level of the FP32 multigrid preconditioner.
 struct MGLevel {
@@ -321,9 +330,36 @@ struct Sim {
     }
 
     Sim();
-    Sim(hipStream_t main, hipStream_t side);
+    Sim(hipStream_t main, hipStream_t side, HostBlock* block);
     ~Sim();
-    int own_streams = 1;
+    Sim(const Sim&) = delete;
+    Sim& operator=(const Sim&) = delete;
+    int own_streams = 1;  // and the host block
+    HostBlock* host = nullptr;
+
+    // ---- device memory ----
+    struct Chunk {
+        char* base = nullptr;
+        size_t size = 0, used = 0;
+        int live = 0;  // allocations in use
+    };
+    static constexpr size_t kMinChunk = 1 << 20;
+    std::vector<Chunk> chunks;
+    char* carve(size_t bytes);
+    void uncarve(void* p);
+    void add_chunk(size_t bytes);
+    void reserve(size_t bytes, int count);
+    void mixed_arrays();
+    // Zeroed device memory for `count` values.
+    template <class T>
+    T* dalloc(long count) {
+        return reinterpret_cast<T*>(carve(sizeof(T) * (size_t)(count > 0 ? count : 1)));
+    }
+    template <class T>
+    void dfree(T*& p) {
+        if (p) uncarve(p);
+        p = nullptr;
+    }
 
     void init_grid(int n, double L, double h, double tol, double eps, double eps_int, int type,
                    int precond);
