@@ -95,10 +95,12 @@ __device__ bool meet(unsigned int* ctl, unsigned int n) {
         if (v >= kPoison) return false;
         const long long now = wall_clock64();
         if (t0 == 0) t0 = now;
-        // Given up, unless the last one arrived just now.
-        if (now - t0 > kWaitTicks)
-            return __hip_atomic_fetch_add(ctl, kPoison, __ATOMIC_RELAXED,
-                                          __HIP_MEMORY_SCOPE_AGENT) == n;
+        // Given up, unless another one arrived just now (the next look tells).
+        unsigned int seen = v;
+        if (now - t0 > kWaitTicks &&
+            __hip_atomic_compare_exchange_strong(ctl, &seen, v + kPoison, __ATOMIC_RELAXED,
+                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            return false;
     }
 }
 
