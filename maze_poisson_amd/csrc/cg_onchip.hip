@@ -858,6 +858,407 @@ __global__ __launch_bounds__(NT) void k_cg_onchip2(Onchip2Args A, PBCoef pb, dou
     }
 }
 
+// ---- larger grids: x and the halo stay in memory -----------------------------------
+// The two-reduction solve of grids whose vectors do not fit whole (about 130^3 to
+// 161^3): r and A p in registers, the own p in LDS without the halo in j and i,
+// which is read from its owner's copy in memory after a third, neighbours-only
+// exchange.  x streams through memory while the sums of the second exchange are
+// on their way.  A work-group holds two tiles of one slab, of the last two slabs
+// where the last is a short one.
+//
+// An iteration moves x (16 B per point), the edges of p (10 B) and the PB
+// coefficients (32 B), where the sweeps move 64 and 128 B: at 160^3 27.6 against
+// 73 us (Poisson) and 44.7 against 117 us (PB; 5.3 TB/s).  The vectors take 144
+// of a thread's 256 registers; batches of more planes than 2 (PB) or 6 (Poisson),
+// whose operands are requested together, spill or give nothing.  Updating x before the second exchange instead of during it costs
+// 2.5 us, half the halo's points in k in registers instead of LDS 4 us (Poisson).
+constexpr int kStreamPlanes = 36;
+constexpr int kStreamStride = kThreads + 4;  // a plane in LDS: p, then the ends of cut rows
+
+struct StreamArgs {
+    GridDims d;
+    int groups, slabs, nwg;  // work-groups per slab, slabs of work-groups, all of them
+    u64* slots;              // a line per work-group: up to four tiles' sums, max|r|, p ready
+    u64* sums;
+    double* h;               // p on the edges, by grid index
+    double* xs;              // x after the first update (x itself is written at the end)
+    unsigned int* ctl;
+    unsigned int epoch;
+};
+constexpr int kReadyWord = 2 * kMaxTiles + 2;
+
+template <bool PB>
+__global__ __launch_bounds__(kThreads) void k_cg_stream(StreamArgs A, PBCoef pb, double* x,
+                                                        const double* r, CGState* st) {
+    constexpr int SLAB = kStreamPlanes, nt = kThreads, LP = kStreamStride, NW = kThreads / kWave;
+    extern __shared__ double lds[];
+    __shared__ double shw[3][NW], sha[4], stops[2];
+    __shared__ int modes[3], bad, ended, result;
+    if (st->done) return;
+    const int n = A.d.n, n2 = A.d.n2, t = threadIdx.x;
+    const int lane = t & (kWave - 1), wv = t / kWave;
+    const int sl = blockIdx.x / A.groups, g0 = blockIdx.x - sl * A.groups;
+    const int base = g0 * nt, cnt = min(nt, n2 - base);
+    const int i0 = sl * A.d.slab, i1 = sl == A.slabs - 1 ? n : i0 + A.d.slab, ni = i1 - i0;
+    const int split = min(ni, A.d.slab);  // planes of the first of up to two slabs
+    const bool act = t < cnt;
+    const int pl = act ? base + t : base;
+    const int idx = pl - base;
+    const int k = pl % n;
+    auto wrap = [n2](int q) { return q < 0 ? q + n2 : q >= n2 ? q - n2 : q; };
+    // Neighbours in j outside the own range come from memory; those in k lie in the
+    // rows the range cuts: its first row's point before the range (LDS entry nt) and
+    // first point (nt + 1), its last row's point after the range and last point.
+    const bool jl = idx < n, jh = idx >= cnt - n;
+    const int jm = wrap(pl - n), jp = wrap(pl + n);
+    const int km = pl + (k == 0 ? n - 1 : -1);
+    const int first = base - base % n, last = base + cnt - 1 - (base + cnt - 1) % n + n - 1;
+    int okm = k == 0 ? n - 1 : -1, okp = k == n - 1 ? 1 - n : 1;
+    if (idx + okm < 0) okm = nt - idx;
+    if (idx + okm >= cnt && k == 0) okm = nt + 3 - idx;
+    if (idx + okp >= cnt) okp = nt + 2 - idx;
+    if (idx + okp < 0) okp = nt + 1 - idx;
+    const int im = (i0 == 0 ? n - 1 : i0 - 1) * n2 + pl;
+    const int ip = (i1 == n ? 0 : i1) * n2 + pl;
+    const bool edge = jl || jh;  // is a neighbour of other work-groups' points
+    const int nb = A.d.blocks;
+    const int tiles = min(2, A.d.chunks - 2 * g0);
+    const double cr = st->plain ? -1.0 : 1.0 / 6.0;
+    double rdv = st->rdv;
+    int iter = 0;
+    unsigned int e = A.epoch;
+    if (t == 0) {
+        bad = ended = 0;
+        stops[0] = st->tol;
+        stops[1] = st->rtol * st->r0;
+        modes[0] = st->limit;
+        modes[1] = st->count_mode;
+        modes[2] = st->plain;
+    }
+
+    const double* xin = x;
+    double R[SLAB], Q[SLAB];
+#pragma unroll
+    for (int u = 0; u < SLAB; u++) {
+        R[u] = r[(i0 + min(u, ni - 1)) * n2 + pl];
+        if (act && u < ni) lds[u * LP + idx] = R[u] * cr;
+    }
+
+    // Tile sums (of two slabs' parts) and max to this work-group's line.
+    auto publish = [&](double s0, double s1, double m, bool with_max) {
+        s0 = wave_sum_rows(s0);
+        s1 = wave_sum_rows(s1);
+        if (with_max) m = wave_max_dpp(m);
+        if (lane == 0) {
+            shw[0][wv] = s0;
+            shw[1][wv] = s1;
+            shw[2][wv] = m;
+        }
+        __syncthreads();
+        if (wv == 0 && lane < kMaxTiles) {
+            const double* w = &shw[lane >> 1][(lane & 1) * (kBlock / kWave)];
+            double v = 0.0;
+            for (int q = 0; q < kBlock / kWave; q++) v += w[q];
+            put(A.slots + kLine * blockIdx.x + 2 * lane, v, e);
+        }
+        if (with_max && wv == 0 && lane == kMaxTiles) {
+            double v = 0.0;
+            for (int w = 0; w < NW; w++) v = fmax(v, shw[2][w]);
+            put(A.slots + kLine * blockIdx.x + 2 * kMaxTiles, v, e);
+        }
+    };
+    // As in k_cg_onchip2; tile (slab, chunk) is part 2 (slab past the last
+    // work-group slab) + chunk & 1 of its work-group.
+    auto offsets = [&](int g, int (&off)[kFoldSlots / kBlock + 1]) {
+#pragma unroll
+        for (int u = 0; u < kFoldSlots / kBlock; u++) {
+            const int xs = g * kWave + lane + u * kBlock;
+            const int tile = xcd_tile(min(xs, nb - 1), nb);
+            const int ts = tile / A.d.chunks, ch = tile - ts * A.d.chunks;
+            const int ws = min(ts, A.slabs - 1);
+            off[u] = xs < nb ? kLine * (ws * A.groups + ch / 2) + 2 * (2 * (ts - ws) + (ch & 1)) : -1;
+        }
+        const int wg = g * kWave + lane;
+        off[kFoldSlots / kBlock] = wg < A.nwg ? kLine * wg + 2 * kMaxTiles : -1;
+    };
+    int mine[kFoldSlots / kBlock + 1];
+    offsets(blockIdx.x, mine);
+    auto fold_groups = [&](bool with_max) {
+        if (wv != 2 || blockIdx.x >= kBlock / kWave) return true;  // (nwg is over 4)
+        double v[kFoldSlots / kBlock + 1];
+        bool ok;
+        if (with_max) {
+            ok = poll_at<kFoldSlots / kBlock + 1>(A.slots, mine, e, A.ctl, v);
+        } else {
+            ok = poll_at<kFoldSlots / kBlock>(A.slots, mine, e, A.ctl, v);
+            v[kFoldSlots / kBlock] = 0.0;
+        }
+        double s = 0.0;
+#pragma unroll
+        for (int u = 0; u < kFoldSlots / kBlock; u++) s += v[u];
+        s = wave_sum_rows(s);
+        const double m = wave_max_dpp(v[kFoldSlots / kBlock]);
+        if (lane == 0) put(A.sums + kLine * blockIdx.x, s, e);
+        if (with_max && lane == 1) put(A.sums + kLine * blockIdx.x + 2, m, e);
+        return ok;
+    };
+    auto totals = [&](bool with_max, double& S, double& M) {
+        const int g = min(lane / 8, kBlock / kWave - 1), c = with_max ? min(lane & 7, 1) : 0;
+        double v[1];
+        const bool ok = poll<1>(A.sums + kLine * g + 2 * c, 0, e, A.ctl, v);
+        S = M = 0.0;
+#pragma unroll
+        for (int q = 0; q < kBlock / kWave; q++) {
+            S += lane_value(v[0], 8 * q);
+            M = fmax(M, with_max ? lane_value(v[0], 8 * q + 1) : 0.0);
+        }
+        return ok;
+    };
+    // The edges of the new p to memory, and the neighbours' (wave 1 waits for the
+    // six work-groups that hold the halo).
+    auto share_p = [&]() {
+        if (act) {
+            const int nu = sopaque(ni);
+            const double* L = lds + vopaque(idx);
+            int c = sopaque(i0) * n2 + vopaque(pl);
+#pragma unroll 4
+            for (int u = 0; u < nu; u++, L += LP, c += n2)
+                if (edge || u == 0 || u == nu - 1) store_partial(A.h, c, L[0]);
+        }
+        __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        bool ok = true;
+        if (wv == 0 && lane == 0) put(A.slots + kLine * blockIdx.x + kReadyWord, 0.0, e);
+        if (wv == 1) {
+            const int q = vopaque(lane);
+            const int p = wrap(q == 2 ? base - n : q == 3 ? base - 1 : q == 4 ? base + cnt
+                                                                              : base + cnt + n - 1);
+            const int s_ = q == 0 ? (sl == 0 ? A.slabs - 1 : sl - 1)
+                                  : q == 1 ? (sl == A.slabs - 1 ? 0 : sl + 1) : sl;
+            const int slot = s_ * A.groups + (q < 2 ? g0 : p / nt);
+            if (q < 6) {
+                double v[1];
+                ok = poll<1>(A.slots + kLine * slot + kReadyWord, 0, e, A.ctl, v);
+            }
+        }
+        // Waves 2 to 4: the ends of cut rows (nothing that is used where a row starts
+        // or ends with the range).
+        const int h = t - 2 * kWave, u = h >> 2;
+        if (h >= 0 && u < ni) {
+            const int q = h & 3, g = q < 2 ? max(g0 - 1, 0) : min(g0 + 1, A.groups - 1);
+            const int p = q == 0 ? max(base - 1, 0) : q == 1 ? first : q == 2 ? min(base + cnt, n2 - 1)
+                                                                              : last;
+            double v[1];
+            ok = poll<1>(A.slots + kLine * (sl * A.groups + g) + kReadyWord, 0, e, A.ctl, v);
+            lds[u * LP + nt + q] = load_partial(A.h, (i0 + u) * n2 + p);
+        }
+        if (!ok) bad = 1;
+        __syncthreads();
+    };
+
+    __syncthreads();
+    e++;
+    share_p();
+    if (bad) return;
+    for (;;) {
+        // A p of the own column and <p, A p>, in batches of planes whose memory
+        // operands are requested together.
+        double s0 = 0.0, s1 = 0.0;
+        {
+            constexpr int UB = PB ? 2 : 6;
+            const int nu = sopaque(ni);
+            const double* L = lds + vopaque(idx);
+            int b0 = sopaque(i0) * n2;
+            double vm = load_partial(A.h, im), vc = L[0];
+            const double vip = load_partial(A.h, ip);
+            double exm = PB ? pb.ex[im] : 0.0;
+#pragma unroll
+            for (int u0 = 0; u0 < SLAB; u0 += UB) {
+                double hjm[UB], hjp[UB];
+                double cx[UB], cy[UB], cz[UB], my[UB], mz[UB], ck[UB];
+                if (u0 < nu) {
+#pragma unroll
+                    for (int u = 0; u < UB; u++) {
+                        const int b = b0 + min(u, nu - 1 - u0) * n2;
+                        hjm[u] = hjp[u] = 0.0;
+                        if (jl) hjm[u] = load_partial(A.h, b + jm);
+                        if (jh) hjp[u] = load_partial(A.h, b + jp);
+                        if (PB) {
+                            cx[u] = pb.ex[b + pl];
+                            cy[u] = pb.ey[b + pl];
+                            cz[u] = pb.ez[b + pl];
+                            my[u] = pb.ey[b + jm];
+                            mz[u] = pb.ez[b + km];
+                            ck[u] = pb.k2[b + pl];
+                        }
+                    }
+#pragma unroll
+                    for (int u = 0; u < UB; u++) {
+                        if (u0 + u < nu) {
+                            const double vp = u0 + u + 1 < nu ? L[LP] : vip;
+                            const double vjm = jl ? hjm[u] : L[jl ? 0 : -n];
+                            const double vjp = jh ? hjp[u] : L[jh ? 0 : n];
+                            const double vkm = L[okm], vkp = L[okp];
+                            double lap;
+                            if (!PB) {
+                                lap = vp + vm + vjp + vjm + vkp + vkm - vc * 6.0;
+                            } else {
+                                lap = vp * cx[u] + vm * exm + vjp * cy[u] + vjm * my[u] +
+                                      vkp * cz[u] + vkm * mz[u] -
+                                      vc * (cx[u] + exm + cy[u] + my[u] + cz[u] + mz[u] + ck[u]);
+                                exm = cx[u];
+                            }
+                            Q[u0 + u] = lap;
+                            const double w = act ? vc * lap : 0.0;
+                            if (u0 + u < split) s0 += w;
+                            else s1 += w;
+                            vm = vc;
+                            vc = vp;
+                        }
+                        L += LP;
+                    }
+                }
+                b0 += UB * n2;
+            }
+        }
+        e++;
+        publish(s0, s1, 0.0, false);
+        // The first planes of x, while the sums are on their way.
+        constexpr int XB = 12;
+        double xv[XB];
+        {
+            const int nu = sopaque(ni), c = sopaque(i0) * n2 + vopaque(pl);
+#pragma unroll
+            for (int u = 0; u < XB; u++) xv[u] = xin[c + min(u, nu - 1) * n2];
+        }
+        bool ok = fold_groups(false);
+        if (wv == 0) {
+            double S, M;
+            ok = totals(false, S, M) && ok;
+            const bool end = fabs(S) < 1e-300;  // breakdown guard, as BodyDir
+            if (lane == 0) {
+                sha[0] = end ? 0.0 : rdv / S;
+                if (end) {
+                    ended = 1;
+                    result = iter;
+                    sha[2] = sha[3] = 0.0;
+                }
+            }
+        }
+        if (!ok) bad = 1;
+        __syncthreads();
+        if (bad) return;
+        if (ended) break;
+        // r += alpha A p, <r, r>, max|r|.
+        const double alpha = sha[0];
+        double m = 0.0;
+        s0 = s1 = 0.0;
+        {
+            const int nu = sopaque(ni);
+#pragma unroll
+            for (int u = 0; u < SLAB; u++) {
+                if (act && u < nu) {
+                    const double rn = R[u] + alpha * Q[u];
+                    R[u] = rn;
+                    if (u < split) s0 += rn * rn;
+                    else s1 += rn * rn;
+                    m = fmax(m, fabs(rn));
+                }
+            }
+        }
+        e++;
+        publish(s0, s1, m, true);
+        ok = fold_groups(true);
+        // x += alpha p, while the sums are on their way.
+        {
+            const int nu = sopaque(ni);
+            const double* L = lds + vopaque(idx);
+            int c = sopaque(i0) * n2 + vopaque(pl);
+#pragma unroll
+            for (int u0 = 0; u0 < SLAB; u0 += XB, c += XB * n2, L += XB * LP) {
+                if (u0 < nu) {
+                    if (u0 > 0) {
+#pragma unroll
+                        for (int u = 0; u < XB; u++) xv[u] = xin[c + min(u, nu - 1 - u0) * n2];
+                    }
+#pragma unroll
+                    for (int u = 0; u < XB; u++)
+                        if (act && u0 + u < nu) A.xs[c + u * n2] = xv[u] + alpha * L[u * LP];
+                }
+            }
+        }
+        xin = A.xs;
+        if (wv == 0) {
+            // The decisions of BodyUpdate::finalize.
+            double S, M, beta = 0.0;
+            ok = totals(true, S, M) && ok;
+            const int limit = modes[0], count = modes[1];
+            int end = 0, res = -1;
+            if (M <= stops[count ? 1 : 0]) {
+                end = 1;
+                res = count ? iter + 1 : iter;
+            } else {
+                const double rn_dot_vn = modes[2] ? S : -S / 6.0;
+                beta = rn_dot_vn / rdv;
+                rdv = rn_dot_vn;
+                if (iter + 1 >= limit) {
+                    end = 1;
+                    res = count ? limit : -1;
+                }
+            }
+            if (lane == 0) {
+                ended = end;
+                result = res;
+                sha[1] = beta;
+                sha[2] = S;
+                sha[3] = M;
+            }
+        }
+        if (!ok) bad = 1;
+        __syncthreads();
+        if (bad) return;
+        if (ended) break;
+        iter++;
+        const double beta = sha[1];
+        {
+            constexpr int UB = 4;
+            const int nu = sopaque(ni);
+            double* L = lds + vopaque(idx);
+#pragma unroll
+            for (int u0 = 0; u0 < SLAB; u0 += UB, L += UB * LP) {
+                if (u0 < nu) {
+                    double v[UB];
+#pragma unroll
+                    for (int u = 0; u < UB; u++) v[u] = L[min(u, nu - 1 - u0) * LP];
+#pragma unroll
+                    for (int u = 0; u < UB; u++)
+                        if (act && u0 + u < nu) L[u * LP] = v[u] * beta + cr * R[u0 + u];
+                }
+            }
+        }
+        e++;
+        share_p();
+        if (bad) return;
+    }
+
+    if (t == 0 && !meet(A.ctl, A.nwg)) bad = 1;
+    __syncthreads();
+    if (bad) return;
+    if (act && xin != x) {
+        int c = i0 * n2 + pl;
+#pragma unroll 4
+        for (int u = 0; u < ni; u++, c += n2) x[c] = xin[c];
+    }
+    if (blockIdx.x == 0 && t == 0) {
+        st->rr = sha[2];
+        st->rmax = sha[3];
+        st->iter = iter;
+        st->first = 0;
+        st->res = result;
+        st->done = 1;
+    }
+}
+
 int slab_class(int slab) {
     return slab <= 1 ? 1 : slab <= 2 ? 2 : slab <= 4 ? 4 : slab <= 8 ? 8 : slab <= 12 ? 12 : 16;
 }
@@ -925,6 +1326,17 @@ void launch2_any(hipStream_t s, const Onchip2Args& a, const PBCoef& pb, double* 
     }
 }
 
+// The work-group slabs of k_cg_stream: the sweeps' own, the last two as one
+// where the chip has no room for a short last one.  0: the grid does not fit.
+int stream_slabs(const GridDims& d, int cus) {
+    const int groups = groups_of(d), last = d.n - (d.slabs - 1) * d.slab;
+    if (d.blocks > kFoldSlots || d.slab > kStreamPlanes) return 0;
+    const bool merge = groups * d.slabs > cus;
+    if (merge && (d.slabs < 2 || d.slab + last > kStreamPlanes)) return 0;
+    const int slabs = d.slabs - (merge ? 1 : 0), nwg = groups * slabs;
+    return nwg <= cus && nwg >= kBlock / kWave ? slabs : 0;
+}
+
 template <bool PB>
 void launch_any(hipStream_t s, const OnchipArgs& a, const PBCoef& pb, double* x, const double* r,
                 CGState* st) {
@@ -981,13 +1393,33 @@ void launch_cg_onchip(hipStream_t s, const GridDims& d, const PBCoef& pb, double
     else launch_any<false>(s, a, pb, x, r, st);
 }
 
-bool cg_onchip2_fits(const GridDims& d) { return tiles_per_wg(d, compute_units()) > 0; }
+bool cg_onchip2_fits(const GridDims& d) {
+    const int cus = compute_units();
+    return tiles_per_wg(d, cus) > 0 || stream_slabs(d, cus) > 0;
+}
 
 void launch_cg_onchip2(hipStream_t s, const GridDims& d, const PBCoef& pb, double* x, double* r,
-                       double* h, CGState* st, const CgOnchip& w) {
+                       double* h, double* xs, CGState* st, const CgOnchip& w) {
     Onchip2Args a;
     a.d = d;
     a.T = tiles_per_wg(d, compute_units());
+    if (!a.T) {
+        StreamArgs b;
+        b.d = d;
+        b.groups = groups_of(d);
+        b.slabs = stream_slabs(d, compute_units());
+        b.nwg = b.groups * b.slabs;
+        b.slots = w.words;
+        b.sums = w.words + (long)kLine * kMaxWg;
+        b.h = h;
+        b.xs = xs;
+        b.ctl = w.ctl;
+        b.epoch = w.epoch;
+        const size_t lds = sizeof(double) * (size_t)kStreamPlanes * kStreamStride;
+        if (pb.ex) MAZE_LAUNCH(k_cg_stream<true>, dim3(b.nwg), dim3(kThreads), lds, s, b, pb, x, r, st);
+        else MAZE_LAUNCH(k_cg_stream<false>, dim3(b.nwg), dim3(kThreads), lds, s, b, pb, x, r, st);
+        return;
+    }
     a.groups = (d.chunks + a.T - 1) / a.T;
     a.nwg = a.groups * d.slabs;
     a.slots = w.words;

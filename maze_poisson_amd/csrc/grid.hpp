@@ -143,10 +143,10 @@ struct CgOnchip {
 GridDims cg_dims_for(int n);
 bool cg_onchip_fits(const GridDims& d);
 // launch_cg_dir / launch_cg_update's solve (two reductions an iteration) likewise,
-// h: one scratch grid; twice the epochs.
+// h, xs: scratch grids; three times the epochs.
 bool cg_onchip2_fits(const GridDims& d);
 void launch_cg_onchip2(hipStream_t s, const GridDims& d, const PBCoef& pb, double* x, double* r,
-                       double* h, CGState* st, const CgOnchip& w);
+                       double* h, double* xs, CGState* st, const CgOnchip& w);
 long cg_onchip_words();
 void launch_cg_onchip(hipStream_t s, const GridDims& d, const PBCoef& pb, double* x, double* r,
                       double* h0, double* h1, CGState* st, const CgOnchip& w);

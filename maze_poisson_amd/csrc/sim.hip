@@ -580,7 +580,7 @@ void Sim::cg_issue(const CgRun& c) {
     if (!cg.onchip)
         cg_chunk();
     else if (cg.two)
-        launch_cg_onchip2(stream, cg.d, cg.pbc, cg.x, cg.rbuf, cg.pin, st, onchip_w);
+        launch_cg_onchip2(stream, cg.d, cg.pbc, cg.x, cg.rbuf, cg.pin, cg.pout, st, onchip_w);
     else
         launch_cg_onchip(stream, cg.d, cg.pbc, cg.x, cg.rbuf, cg.pin, cg.pout, st, onchip_w);
     publish();
@@ -596,7 +596,7 @@ bool Sim::onchip_next(const GridDims& d, int limit, int two) {
     // Per-kernel timing names the sweeps, so it runs them.
     if (!onchip || prof || !(two ? cg_onchip2_fits(d) : cg_onchip_fits(d))) return false;
     const long words = cg_onchip_words();
-    const unsigned int span = 2u * (unsigned int)limit + 4u;
+    const unsigned int span = 3u * (unsigned int)limit + 6u;
     if (!onchip_w.words) {
         onchip_w.words = dalloc<unsigned long long>(words);
         onchip_w.ctl = dalloc<unsigned int>(1);

@@ -54,6 +54,28 @@ def test_onchip_pb_cg_equals_sweeps(hip_raw, n, reductions):
     assert np.array_equal(xo, xs)
 
 
+# Grids whose x and halo stay in memory: last slabs whole and merged with the one
+# before, last work-groups that are nearly full and far smaller than a row, rows that
+# start at every offset to a work-group's range.
+STREAM_MAX = 161
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pb", [0, 1])
+@pytest.mark.parametrize("n", [130, 131, 134, 143, 145, 160, STREAM_MAX])
+def test_streaming_cg_equals_sweeps(hip_raw, n, pb):
+    b, x0 = _problem(n, n)
+    g = np.random.default_rng(7)
+    coef = [g.uniform(2.0, 80.0, (n, n, n)) for _ in range(3)] + [g.uniform(0.0, 0.1, (n, n, n))]
+    coef = coef if pb else None
+    tol = 1e-4 * np.abs(b).max()
+    xs, xo = x0.copy(), x0.copy()
+    i_s = _solve(hip_raw, b, xs, tol, n, 2, 0, coef)
+    i_o = _solve(hip_raw, b, xo, tol, n, 2, 1, coef)
+    assert i_o == i_s and i_s >= 0
+    assert np.array_equal(xo, xs)
+
+
 # The one-reduction recurrence against the two-reduction one: the same iterates up to
 # rounding.  A relative difference of 1e-16 per sum stays within 1e-10 of the solution
 # over a solve of under 300 iterations.
@@ -72,7 +94,7 @@ def test_one_reduction_equals_two(hip_raw, n):
 @pytest.mark.gpu
 @pytest.mark.parametrize("reductions", [1, 2])
 def test_onchip_cg_limits(hip_raw, reductions):
-    n = FIT_MAX + 2
+    n = (FIT_MAX if reductions == 1 else STREAM_MAX) + 2
     b, x = _problem(n, 1)
     assert _solve(hip_raw, b, x, 1.0, n, reductions, 1) == -2
     # A zero residual stops before the first direction, with x unchanged.
@@ -89,9 +111,8 @@ def test_onchip_cg_limits(hip_raw, reductions):
 
 # A launch that finds its solve abandoned leaves x alone, and the sweeps run it.
 @pytest.mark.gpu
-@pytest.mark.parametrize("reductions", [1, 2])
-def test_abandoned_launch_falls_back(hip_raw, reductions):
-    n = 64
+@pytest.mark.parametrize("n,reductions", [(64, 1), (64, 2), (134, 2)])
+def test_abandoned_launch_falls_back(hip_raw, n, reductions):
     b, x0 = _problem(n, 3)
     tol = 1e-6 * np.abs(b).max()
     xs, xo = x0.copy(), x0.copy()
