@@ -108,17 +108,6 @@ __device__ __forceinline__ double cube(double x) {
     return fma(hi, x, lo * x);
 }
 
-// First index in the ascending a[0..n) whose value is >= key.
-__device__ __forceinline__ int lower_bound_u32(const unsigned int* a, int n, unsigned int key) {
-    int lo = 0, hi = n;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (a[mid] < key) lo = mid + 1;
-        else hi = mid;
-    }
-    return lo;
-}
-
 // Neighbour offsets of a point inside its i-plane (periodic in j and k).
 struct PlaneNb {
     int jm, jp, km, kp;

@@ -152,14 +152,11 @@ static long long arena_bytes(int n, int np, int precision, const Phys& ph) {
     b += 8 * G;                                           // spread list heads
     b += 8LL * tf_part_doubles(np) + 7LL * 8 * 16 * 16;  // pair table, up to 16 types
     if (ph.pb == 2) {
-        // radii, squared reach, map / force reach, bin keys and ids (sorted and
-        // not), the three boundary forces, the key sort's work space
-        const int nb = (n + kPbTile - 1) / kPbTile;
-        const unsigned long bins = (unsigned long)nb * nb * nb;
-        int key_bits = 1;
-        while ((1ul << key_bits) < bins) key_bits++;
-        b += (long long)np * (3 * 8 + 2 * 4 + 4 * 4 + 3 * 24);
-        b += (long long)std::max<size_t>(pb_sort_bytes(std::max(np, 1), key_bits), 16);
+        // radii, squared reach, map / force reach, the ion lists of the bins, the
+        // marks of the maps, the three boundary forces
+        const long long nb = (n + kPbTile - 1) / kPbTile;
+        b += (long long)np * (3 * 8 + 2 * 4 + 4 + 3 * 24) + 4 * nb * nb * nb + G;
+        b += 8LL * n * n * ((n + kWave - 1) / kWave);
         allocs += 16;
     }
     return b + (long long)allocs * (long long)kArenaAlign;  // alignment of each allocation

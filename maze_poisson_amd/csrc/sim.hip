@@ -230,10 +230,9 @@ void Sim::free_particles() {
 
 void Sim::free_pb() {
     for (double** a : {&pbd.radii, &pbd.rp2, &pbd.rm2, &pbd.fdb, &pbd.fib, &pbd.fnp}) dfree(*a);
-    for (int** a : {&pbd.rmap, &pbd.rfrc, &pbd.ids, &pbd.ids_sorted}) dfree(*a);
-    dfree(pbd.keys);
-    dfree(pbd.keys_sorted);
-    dfree(pbd.sort_tmp);
+    for (int** a : {&pbd.rmap, &pbd.rfrc, &pbd.head, &pbd.next}) dfree(*a);
+    dfree(pbd.mark);
+    dfree(pbd.any);
     pbd = PBDev{};
     pb_flag_pending = 0;
 }
@@ -300,6 +299,7 @@ void Sim::init_grid(int n_, double L_, double h_, double tol_, double eps, doubl
 // library/src/grid_general.c:85-100 (maps default to vacuum until set).
 void Sim::init_pb(double w_, double kbar2_, int nonpolar_) {
     pb = 1; w = w_; kbar2 = kbar2_; nonpolar = nonpolar_;
+    pbd.marked = 0;
     pbmg_dirty = 1;
     reserve(4 * sizeof(double) * (size_t)G, 4);
     ex = dalloc<double>(G); ey = dalloc<double>(G); ez = dalloc<double>(G); k2 = dalloc<double>(G);
@@ -313,6 +313,7 @@ void Sim::init_pb(double w_, double kbar2_, int nonpolar_) {
 
 void Sim::set_eps_k2(const double* ex_, const double* ey_, const double* ez_, const double* k2_) {
     pbmg_dirty = 1;
+    pbd.marked = 0;
     if (!pb) fatal("maze: solver_set_eps_k2 needs solver_initialize_grid_pois_boltz first");
     MAZE_HIP(hipMemcpy(ex, ex_, G * sizeof(double), hipMemcpyHostToDevice));
     MAZE_HIP(hipMemcpy(ey, ey_, G * sizeof(double), hipMemcpyHostToDevice));
@@ -405,17 +406,14 @@ void Sim::init_pb_particles(double gamma_np, double beta_np, const double* radii
     }
     pbd.rmax = rmax;
     pbd.nb = (n + kPbTile - 1) / kPbTile;
-    const unsigned long bins = (unsigned long)pbd.nb * pbd.nb * pbd.nb;
-    pbd.key_bits = 1;
-    while ((1ul << pbd.key_bits) < bins) pbd.key_bits++;
     pbd.radii = dalloc<double>(np); pbd.rp2 = dalloc<double>(np); pbd.rm2 = dalloc<double>(np);
     pbd.rmap = dalloc<int>(np); pbd.rfrc = dalloc<int>(np);
-    pbd.keys = dalloc<unsigned int>(np); pbd.keys_sorted = dalloc<unsigned int>(np);
-    pbd.ids = dalloc<int>(np); pbd.ids_sorted = dalloc<int>(np);
+    pbd.head = dalloc<int>((long)pbd.nb * pbd.nb * pbd.nb); pbd.next = dalloc<int>(np);
+    pbd.mark = dalloc<unsigned char>(G);
+    pbd.words = (n + kWave - 1) / kWave;
+    pbd.any = dalloc<unsigned long long>((long)n * n * pbd.words);
     pbd.fdb = dalloc<double>(3L * np); pbd.fib = dalloc<double>(3L * np);
     pbd.fnp = dalloc<double>(3L * np);
-    pbd.sort_bytes = pb_sort_bytes(std::max(np, 1), pbd.key_bits);
-    pbd.sort_tmp = dalloc<char>((long)std::max<size_t>(pbd.sort_bytes, 16));
     pbd.flag = &ps->pb_flag;
     if (np > 0) {
         MAZE_HIP(hipMemcpy(pbd.radii, radii, np * sizeof(double), hipMemcpyHostToDevice));
@@ -456,6 +454,7 @@ double Sim::forces_pb() {
     if (!pbd.active)
         fatal("maze: PB boundary forces need the ion radii (solver_initialize_particles_pois_boltz)");
     check_pb_flag();
+    launch_pb_any(stream, pbd, ex, ey, ez, k2);
     timed(kTPbForces, 0, [&] { launch_pb_forces(stream, pbd, p.pos, phi, ex, ey, ez, k2); });
     return 0.0;
 }

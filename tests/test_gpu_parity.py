@@ -846,6 +846,38 @@ def test_pb_forces_match_oracle(hip, oracle, name, nonpolar):
         assert np.abs(g[k] - o[k]).max() <= 1e-12 * scale, (k, np.abs(g[k] - o[k]).max() / scale)
 
 
+# Grids of one to a few partly filled 8^3 tiles whose bins all reach each other, more
+# than 128 ions within reach of a tile, spheres smaller than the transition width, ions
+# on cell borders.  Maps: with s^3 rounded differently, a shell factor c3 s^3 + c2 s^2 in
+# (0, 1] with |c3 s^3| <= 2 differs by up to 2 + 2 + 1 units and its product by one more;
+# 6 * 2^-53 for each of up to 8 shells.
+@pytest.mark.parametrize("n_ions,n,w,radii", [(8, 13, 0.5, (0.3, 0.6)), (8, 23, 2.9, (0.0, 0.2)),
+                                              (512, 20, 1.0, (2.5, 4.0)),
+                                              (64, 33, 1.5, (0.4, 2.5))])
+def test_pb_radii_edges_match_oracle(hip, oracle, n_ions, n, w, radii):
+    phi = np.random.default_rng(5).normal(size=(n, n, n))
+    res = []
+    for lib in (hip, oracle):
+        s = W.nacl_system(n_ions, n, seed=9)
+        s.pos[0] = 0.0
+        s.pos[1] = [s.h, 2 * s.h, s.L - s.h]
+        cfg = driver.RunConfig(tol=W.poisson_tol(s), eps_s=80.0, pb_radii=True, pb_w=w,
+                               radii_ang=radii, probe_ang=0.3, nonpolar=True, gamma_np=0.05)
+        driver.initialize(lib, s, cfg)
+        lib.solver_update_charges()
+        lib.solver_update_eps_k2()
+        lib.solver_set_field(phi)
+        lib.solver_compute_forces_pb()
+        out = get_maps(lib, n)
+        for k in ("db", "ib", "np"):
+            out.append(np.zeros((n_ions, 3)))
+            getattr(lib, "get_fcs_" + k)(out[-1])
+        res.append(out)
+        lib.solver_finalize()
+    for q, (g, o) in enumerate(zip(*res)):
+        assert np.abs(g - o).max() <= (48 * 2.0**-53 if q < 4 else 1e-12) * np.abs(o).max(), q
+
+
 @pytest.mark.parametrize("method", ["MAZE-LCG", "LCG", "MULTIGRID", "MAZE-MULTIGRID"])
 def test_md_sequence_pb_radii(hip, oracle, method):
     """MD steps with the radius-based PB boundary rebuilt every step and its forces in
