@@ -2,6 +2,8 @@
 in seconds).  Point-wise kernels must agree bit for bit (they follow the reference's
 operation order); anything that goes through a global sum (CG scalars) agrees to
 the stated tolerances.  Every test calls the product through its C-ABI."""
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -760,6 +762,52 @@ def test_field_matches_fft_poisson_at_128(hip, precision):
     phi = np.fft.ifftn(ph).real
     d = (g["field"] - g["field"].mean()) - phi
     assert np.abs(d).max() <= 1e-6 * np.abs(phi).max(), np.abs(d).max() / np.abs(phi).max()
+
+
+# Blocks of 64 ions as clusters, some further apart than the cutoff and some across the
+# box border, a last block that is full, nearly empty or nearly full, one block only;
+# the pair table in LDS and in memory.  A pair term is within 60 roundings on either
+# side and a sum has up to n_p of them.
+@pytest.mark.parametrize("n_typ", [2, 5])
+@pytest.mark.parametrize("n_p", [2, 63, 64, 65, 320, 383])
+def test_tf_blocks_match_oracle(hip, oracle, oracle_raw, n_p, n_typ):
+    g = np.random.default_rng(n_p + n_typ)
+    s = W.nacl_system(216, 32, seed=1)
+    L, rc = s.L, s.L / 2
+    lat = np.array([(i, j, k) for i in range(4) for j in range(4) for k in range(4)]) * 2.0
+    at = [(0, 0, 0), (.5, 0, 0), (0, .5, .5), (.5, .5, 0), (.45, .5, .5), (.5, 0, .5)]
+    pos = np.concatenate([lat + np.array(c) * L for c in at]) + g.uniform(-.2, .2, (384, 3))
+    pos = np.ascontiguousarray((pos % L)[:n_p])
+    types = g.integers(0, n_typ, n_p).astype(np.int32)
+    tf = np.tile(s.tf.reshape(-1, 5)[1], (n_typ, n_typ, 1))
+    tf[..., 0] *= 1 + 0.1 * (np.arange(n_typ)[:, None] + np.arange(n_typ))
+    s = dataclasses.replace(s, n_typ=n_typ, types=types, pos=pos, vel=np.zeros((n_p, 3)),
+                            mass=np.ones(n_p), charges=np.where(np.arange(n_p) % 2, 1.0, -1.0),
+                            tf=tf.ravel())
+    out = []
+    for lib in (hip, oracle):
+        driver.initialize(lib, s, driver.RunConfig(tol=1.0))
+        v = lib.solver_compute_forces_noel()
+        f, cnt = np.zeros((n_p, 3)), np.zeros(n_p, dtype=np.int32)
+        lib.get_fcs_noel(f)
+        lib.get_tf_neighbor_counts(cnt)
+        out.append((v, f, cnt))
+        lib.solver_finalize()
+    table = np.zeros(n_typ * n_typ * 7)
+    oracle_raw.or_tf_pair_table(n_typ, s.tf, rc, table)
+    a, b, c, d, sg, al, be = table.reshape(-1, 7)[types[:, None] * n_typ + types].transpose(2, 0, 1)
+    x = pos[:, None] - pos
+    x -= L * np.round(x / L)
+    r = np.sqrt((x ** 2).sum(-1)) + 1e9 * np.eye(n_p)
+    ex = a * np.exp(b * (sg - r))
+    near = r <= rc
+    fm = (b * ex + 6 * abs(c) / r ** 7 + 8 * abs(d) / r ** 9 + abs(al)) * near
+    vm = (ex + abs(c) / r ** 6 + abs(d) / r ** 8 + abs(al) * r + abs(be)) * near
+    (v, f, cnt), (vo, fo, co) = out
+    assert np.array_equal(cnt, co) and np.array_equal(cnt, near.sum(1))
+    u = (120 + 2 * n_p) * 2.0 ** -53
+    assert (np.abs(f - fo) <= u * fm.sum(1)[:, None]).all()
+    assert abs(v - vo) <= u * vm.sum()
 
 
 # ---- Poisson-Boltzmann boundary from ion radii -------------------------------------
