@@ -49,6 +49,7 @@ double quantile(std::vector<double> v, double q) {
 struct Lane {
     hipStream_t main = nullptr, side = nullptr;
     HostBlock* host = nullptr;
+    bool wide = false;  // from Engine::wide_pool
 };
 
 // Physics of a request beyond maze_engine_submit's defaults (MAZE-LCG without
@@ -203,7 +204,7 @@ struct Engine {
     // Streams and pinned blocks of retired replicas, reused by the next ones
     // (creating a stream costs milliseconds, freeing a pinned block 0.2 ms);
     // destroyed with the engine.
-    std::vector<Lane> lane_pool;
+    std::vector<Lane> lane_pool, wide_pool;
 
     // New streams come Q main streams, then their Q side streams, Q being the
     // runtime's hardware queues per process (GPU_MAX_HW_QUEUES, four by
@@ -211,39 +212,48 @@ struct Engine {
     // replicas' solve streams spread over all queues instead of alternating
     // with the short pair-force streams. The pool so holds at most Q - 1 idle
     // pairs beyond those of the replicas that ever ran at once.
+    // A lane's two streams so mostly share a queue: its pair forces run between its
+    // solves, beside those of others (32 replicas 283 ms; 290 with the pair forces of
+    // one replica on the queue of another's solve).  A replica whose pair kernel is
+    // made to run beside its own solve (`wide`, tf_beside) takes two streams made one
+    // right after the other, which go to different queues: 32768 ions on 256^3 153 ms
+    // for 40 steps, 188 on one queue.
     // `created` gets the drop of free device memory over a new batch: the
     // runtime sets up its hardware queues (a per-process cost, at most four
     // queues) as the first streams are made, so it is not a per-replica cost.
-    Lane take_lane(long long& created) {
+    Lane take_lane(long long& created, bool wide) {
         created = 0;
         std::lock_guard<std::mutex> g(mu);
-        if (lane_pool.empty()) {
-            const int q = hw_queues();
+        std::vector<Lane>& pool = wide ? wide_pool : lane_pool;
+        if (pool.empty()) {
+            const int q = wide ? 1 : hw_queues();
             size_t f0 = 0, f1 = 0, total = 0;
             MAZE_HIP(hipMemGetInfo(&f0, &total));
             std::vector<hipStream_t> mains(q), sides(q);
             for (auto& m : mains) MAZE_HIP(hipStreamCreateWithFlags(&m, hipStreamNonBlocking));
             for (auto& sd : sides) MAZE_HIP(hipStreamCreateWithFlags(&sd, hipStreamNonBlocking));
             for (int k = q - 1; k >= 0; k--)
-                lane_pool.push_back({mains[k], sides[k], host_block_create()});
+                pool.push_back({mains[k], sides[k], host_block_create(), wide});
             MAZE_HIP(hipMemGetInfo(&f1, &total));
             created = (long long)f0 - (long long)f1;
         }
-        const Lane l = lane_pool.back();
-        lane_pool.pop_back();
+        const Lane l = pool.back();
+        pool.pop_back();
         return l;
     }
 
     void give_lane(const Lane& l) {
         std::lock_guard<std::mutex> g(mu);
-        lane_pool.push_back(l);
+        (l.wide ? wide_pool : lane_pool).push_back(l);
     }
 
     ~Engine() {
-        for (Lane& l : lane_pool) {
-            MAZE_HIP(hipStreamDestroy(l.main));
-            MAZE_HIP(hipStreamDestroy(l.side));
-            host_block_destroy(l.host);
+        for (const std::vector<Lane>* pool : {&lane_pool, &wide_pool}) {
+            for (const Lane& l : *pool) {
+                MAZE_HIP(hipStreamDestroy(l.main));
+                MAZE_HIP(hipStreamDestroy(l.side));
+                host_block_destroy(l.host);
+            }
         }
     }
 
@@ -253,7 +263,7 @@ struct Engine {
         r.used_precision = precision_for(r.n, r.precision, r.ph);
         // Its lane comes from the pool, created four at a time and counted apart
         // from the replica's own memory.
-        r.lane = take_lane(r.stream_bytes);
+        r.lane = take_lane(r.stream_bytes, tf_beside(r.n, r.np));
         size_t free0 = 0, total = 0;
         MAZE_HIP(hipMemGetInfo(&free0, &total));
         r.arena = std::make_unique<DevArena>();

@@ -6,6 +6,7 @@
 // library/src/integrator_ovrvo.c:45-123) so that per-ion results match the
 // CPU oracle bit for bit wherever no transcendental function is involved.
 
+#include "grid.hpp"
 #include "particles.hpp"
 
 namespace maze {
@@ -351,12 +352,14 @@ void launch_force_fd_kick(hipStream_t s, const PDev& p, const double* phi, doubl
 // kept short: both roots from one reciprocal square root, products of the pair
 // coefficients formed once, LDS adds without a return, pairs counted in ballots, no
 // bounds checks in full blocks.  Blocks whose extents lie further apart than the
-// cutoff are skipped.  32768 ions 1.94 ms (2.14 with the library's root, division and
+// cutoff are skipped.  Fewer work-groups than block pairs take theirs from a queue
+// (tf_beside).  32768 ions 1.94 ms (2.14 with the library's root, division and
 // rounding), 4096 50 us (56), 216 10.9 us (12.6); the sums keep their order and bits.
 constexpr int kTfB = 64;
 constexpr int kTfWaves = 4;
+constexpr int kTfCus = 256;
 
-__device__ __forceinline__ int tf_item(int I, int J, int nb) { return I * nb - I * (I - 1) / 2 + (J - I); }
+__host__ __device__ __forceinline__ int tf_item(int I, int J, int nb) { return I * nb - I * (I - 1) / 2 + (J - I); }
 
 // The type-pair table sits in LDS for up to kTfLdsTypes types, else it is
 // read from global memory.
@@ -400,131 +403,154 @@ template <bool LdsTab>
 __global__ __launch_bounds__(kTfB * kTfWaves) void k_tf_tiles(
     int np, int n_typ, double L, double invL, double r_cut, const double* __restrict__ pos,
     const int* __restrict__ types, const double* __restrict__ table, double* __restrict__ part,
-    int i_off) {
-    const int J = blockIdx.x, I = blockIdx.y + i_off, nb = gridDim.x;
-    if (I > J) return;
+    unsigned int* queue) {
     __shared__ double sx[kTfB], sy[kTfB], sz[kTfB], gap[3];
-    __shared__ int styp[kTfB];
+    __shared__ int styp[kTfB], next;
     __shared__ double acc[kTfWaves][4][kTfB];  // j-role, per wave
     __shared__ double own[kTfWaves][4][kTfB];  // i-role, per wave
     __shared__ int met[kTfWaves][2 * kTfB];    // pairs, i-role then j-role
     __shared__ TfPair tab[LdsTab ? kTfLdsTypes * kTfLdsTypes : 1];
     const int tid = threadIdx.x, l = tid & (kTfB - 1), w = tid / kTfB;
     if (LdsTab && tid < n_typ * n_typ) tab[tid] = tf_pair(table + 7 * tid);
-    const int jl = J * kTfB + l;
-    const bool jv = jl < np;
-    if (w == 0) {
-        sx[l] = jv ? pos[3 * jl] : 0.0;
-        sy[l] = jv ? pos[3 * jl + 1] : 0.0;
-        sz[l] = jv ? pos[3 * jl + 2] : 0.0;
-        styp[l] = jv ? types[jl] : 0;
-    }
-    for (int c = 0; c < 4; c++) acc[w][c][l] = 0.0;
-    const int i = I * kTfB + l;
-    const bool iv = i < np;
-    const double xi = iv ? pos[3 * i] : 0.0, yi = iv ? pos[3 * i + 1] : 0.0,
-                 zi = iv ? pos[3 * i + 2] : 0.0;
-    const int ti = (iv ? types[i] : 0) * n_typ;
-    __syncthreads();
-    const bool diag = I == J;
-    // The blocks' distance along axis w: each block's extent around its first ion.
-    if (w < 3 && !diag) {
-        const double a = w == 0 ? xi : w == 1 ? yi : zi;
-        const double b = w == 0 ? sx[l] : w == 1 ? sy[l] : sz[l];
-        auto image = [&](double d) { return d - L * round_away(d * invL); };
-        const double a0 = lane_value(a, 0), b0 = lane_value(b, 0);
-        const double da = iv ? image(a - a0) : 0.0, db = jv ? image(b - b0) : 0.0;
-        const double D = image(b0 - a0);
-        const double lo = D - wave_max_dpp(-db) - wave_max_dpp(da);
-        const double hi = D + wave_max_dpp(db) + wave_max_dpp(-da);
-        double g = fmax(fmax(lo, -hi), 0.0);
-        g = fmin(g, fmax(fmax(lo - L, L - hi), 0.0));
-        g = fmin(g, fmax(fmax(lo + L, -L - hi), 0.0));
-        if (l == 0) gap[w] = g;
-    }
-    double f0 = 0.0, f1 = 0.0, f2 = 0.0, e = 0.0;
-    int mi = 0, mj = 0;
-    // Waves share only the read-only j block; each accumulates reactions in its
-    // own LDS rows, and within a wave the lanes of one step touch distinct j and
-    // successive steps are in program order, so the steps need no barrier.
-    auto step = [&](int s, bool ok) {
-        const int jj = (l + s) & (kTfB - 1);
-        double app = xi - sx[jj];
-        app -= L * round_away(app * invL);
-        double r2 = app * app;
-        const double d0 = app;
-        app = yi - sy[jj];
-        app -= L * round_away(app * invL);
-        const double d1 = app;
-        r2 += app * app;
-        app = zi - sz[jj];
-        app -= L * round_away(app * invL);
-        const double d2 = app;
-        r2 += app * app;
-        double r, ir;
-        root(r2, r, ir);
-        if (!(r2 > 1e-200 && r2 < 1e200)) {  // coincident ions, positions not finite
-            r = sqrt(r2);
-            ir = 1.0 / r;
+    const int nb = (np + kTfB - 1) / kTfB, items = tf_item(nb, nb, nb);
+    const bool queued = (int)gridDim.x < items;
+    for (int item = blockIdx.x; item < items;) {
+        // The next item's number is on its way while this one is evaluated.
+        unsigned int ticket = 0;
+        if (queued && tid == 0)
+            ticket = __hip_atomic_fetch_add(queue, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // Row I starts at item I nb - I (I - 1) / 2.
+        int I = (int)(nb + 0.5f - sqrtf(fmaxf((nb + 0.5f) * (nb + 0.5f) - 2.0f * item, 0.0f)));
+        I = max(min(I, nb - 1), 0);
+        while (I > 0 && tf_item(I, I, nb) > item) I--;
+        while (tf_item(I + 1, I + 1, nb) <= item) I++;
+        const int J = I + item - tf_item(I, I, nb);
+        const int jl = J * kTfB + l;
+        const bool jv = jl < np;
+        if (w == 0) {
+            sx[l] = jv ? pos[3 * jl] : 0.0;
+            sy[l] = jv ? pos[3 * jl + 1] : 0.0;
+            sz[l] = jv ? pos[3 * jl + 2] : 0.0;
+            styp[l] = jv ? types[jl] : 0;
         }
-        ok = ok && r <= r_cut;
-        const unsigned long long m = __ballot(ok);
-        mi += ok;
-        mj += __builtin_amdgcn_inverse_ballot_w64(s == 0 ? m : m << s | m >> (kTfB - s));
-        if (ok) {
-            const TfPair t = LdsTab ? tab[ti + styp[jj]] : tf_pair(table + 7 * (ti + styp[jj]));
-            const double ex = exp(t.b * (t.sg - r));
-            const double ir2 = ir * ir;
-            const double ir6 = ir2 * ir2 * ir2;
-            const double ir8 = ir6 * ir2;
-            const double fm = t.ba * ex - t.c6 * (ir6 * ir) - t.d8 * (ir8 * ir) - t.al;
-            const double vm = t.a * ex - t.c * ir6 - t.d * ir8 + t.al * r + t.be;
-            // The force on j; that on i is its opposite.
-            const double g0 = -fm * (d0 * ir), g1 = -fm * (d1 * ir), g2 = -fm * (d2 * ir);
-            f0 -= g0;
-            f1 -= g1;
-            f2 -= g2;
-            e += vm;
-            unsafeAtomicAdd(&acc[w][0][jj], g0);
-            unsafeAtomicAdd(&acc[w][1][jj], g1);
-            unsafeAtomicAdd(&acc[w][2][jj], g2);
-            unsafeAtomicAdd(&acc[w][3][jj], vm);
+        for (int c = 0; c < 4; c++) acc[w][c][l] = 0.0;
+        const int i = I * kTfB + l;
+        const bool iv = i < np;
+        const double xi = iv ? pos[3 * i] : 0.0, yi = iv ? pos[3 * i + 1] : 0.0,
+                     zi = iv ? pos[3 * i + 2] : 0.0;
+        const int ti = (iv ? types[i] : 0) * n_typ;
+        __syncthreads();
+        const bool diag = I == J;
+        // The blocks' distance along axis w: each block's extent around its first ion.
+        if (w < 3 && !diag) {
+            const double a = w == 0 ? xi : w == 1 ? yi : zi;
+            const double b = w == 0 ? sx[l] : w == 1 ? sy[l] : sz[l];
+            auto image = [&](double d) { return d - L * round_away(d * invL); };
+            const double a0 = lane_value(a, 0), b0 = lane_value(b, 0);
+            const double da = iv ? image(a - a0) : 0.0, db = jv ? image(b - b0) : 0.0;
+            const double D = image(b0 - a0);
+            const double lo = D - wave_max_dpp(-db) - wave_max_dpp(da);
+            const double hi = D + wave_max_dpp(db) + wave_max_dpp(-da);
+            double g = fmax(fmax(lo, -hi), 0.0);
+            g = fmin(g, fmax(fmax(lo - L, L - hi), 0.0));
+            g = fmin(g, fmax(fmax(lo + L, -L - hi), 0.0));
+            if (l == 0) gap[w] = g;
         }
-    };
-    __syncthreads();
-    if (diag) {
-        for (int s = 1 + w; s <= 32; s += kTfWaves)
-            step(s, iv && I * kTfB + ((l + s) & (kTfB - 1)) < np && !(s == 32 && l >= 32));
-    } else if (!(gap[0] * gap[0] + gap[1] * gap[1] + gap[2] * gap[2] >
-                 r_cut * r_cut * (1.0 + 1e-9))) {
-        if (J * kTfB + kTfB <= np)
-            for (int s = w; s < kTfB; s += kTfWaves) step(s, true);
-        else
-            for (int s = w; s < kTfB; s += kTfWaves)
-                step(s, J * kTfB + ((l + s) & (kTfB - 1)) < np);
+        double f0 = 0.0, f1 = 0.0, f2 = 0.0, e = 0.0;
+        int mi = 0, mj = 0;
+        // Waves share only the read-only j block; each accumulates reactions in its
+        // own LDS rows, and within a wave the lanes of one step touch distinct j and
+        // successive steps are in program order, so the steps need no barrier.
+        auto step = [&](int s, bool ok) {
+            const int jj = (l + s) & (kTfB - 1);
+            double app = xi - sx[jj];
+            app -= L * round_away(app * invL);
+            double r2 = app * app;
+            const double d0 = app;
+            app = yi - sy[jj];
+            app -= L * round_away(app * invL);
+            const double d1 = app;
+            r2 += app * app;
+            app = zi - sz[jj];
+            app -= L * round_away(app * invL);
+            const double d2 = app;
+            r2 += app * app;
+            double r, ir;
+            root(r2, r, ir);
+            if (!(r2 > 1e-200 && r2 < 1e200)) {  // coincident ions, positions not finite
+                r = sqrt(r2);
+                ir = 1.0 / r;
+            }
+            ok = ok && r <= r_cut;
+            const unsigned long long m = __ballot(ok);
+            mi += ok;
+            mj += __builtin_amdgcn_inverse_ballot_w64(s == 0 ? m : m << s | m >> (kTfB - s));
+            if (ok) {
+                const TfPair t = LdsTab ? tab[ti + styp[jj]] : tf_pair(table + 7 * (ti + styp[jj]));
+                const double ex = exp(t.b * (t.sg - r));
+                const double ir2 = ir * ir;
+                const double ir6 = ir2 * ir2 * ir2;
+                const double ir8 = ir6 * ir2;
+                const double fm = t.ba * ex - t.c6 * (ir6 * ir) - t.d8 * (ir8 * ir) - t.al;
+                const double vm = t.a * ex - t.c * ir6 - t.d * ir8 + t.al * r + t.be;
+                // The force on j; that on i is its opposite.
+                const double g0 = -fm * (d0 * ir), g1 = -fm * (d1 * ir), g2 = -fm * (d2 * ir);
+                f0 -= g0;
+                f1 -= g1;
+                f2 -= g2;
+                e += vm;
+                unsafeAtomicAdd(&acc[w][0][jj], g0);
+                unsafeAtomicAdd(&acc[w][1][jj], g1);
+                unsafeAtomicAdd(&acc[w][2][jj], g2);
+                unsafeAtomicAdd(&acc[w][3][jj], vm);
+            }
+        };
+        __syncthreads();
+        if (diag) {
+            for (int s = 1 + w; s <= 32; s += kTfWaves)
+                step(s, iv && I * kTfB + ((l + s) & (kTfB - 1)) < np && !(s == 32 && l >= 32));
+        } else if (!(gap[0] * gap[0] + gap[1] * gap[1] + gap[2] * gap[2] >
+                     r_cut * r_cut * (1.0 + 1e-9))) {
+            if (J * kTfB + kTfB <= np)
+                for (int s = w; s < kTfB; s += kTfWaves) step(s, true);
+            else
+                for (int s = w; s < kTfB; s += kTfWaves)
+                    step(s, J * kTfB + ((l + s) & (kTfB - 1)) < np);
+        }
+        own[w][0][l] = f0;
+        own[w][1][l] = f1;
+        own[w][2][l] = f2;
+        own[w][3][l] = e;
+        met[w][l] = mi;
+        met[w][kTfB + l] = mj;
+        __syncthreads();
+        // part[item][component][slot]: slots 0..63 the i-role, 64..127 the j-role.
+        double* o = part + (long)item * 5 * 2 * kTfB;
+        for (int x = tid; x < 5 * 2 * kTfB; x += kTfB * kTfWaves) {
+            const int c = x / (2 * kTfB), slot = x % (2 * kTfB);
+            const bool jr = slot >= kTfB;
+            const int q = jr ? slot - kTfB : slot;
+            double v = 0.0;
+            if (c < 4) {
+                for (int u = 0; u < kTfWaves; u++) v += jr ? acc[u][c][q] : own[u][c][q];
+            } else {
+                int k = 0;
+                for (int u = 0; u < kTfWaves; u++) k += met[u][slot];
+                v = k;
+            }
+            o[x] = v;
+        }
+        if (!queued) break;
+        if (tid == 0) next = gridDim.x + ticket;
+        __syncthreads();
+        item = next;
     }
-    own[w][0][l] = f0;
-    own[w][1][l] = f1;
-    own[w][2][l] = f2;
-    own[w][3][l] = e;
-    met[w][l] = mi;
-    met[w][kTfB + l] = mj;
-    __syncthreads();
-    // part[item][component][slot]: slots 0..63 the i-role, 64..127 the j-role.
-    double* o = part + (long)tf_item(I, J, nb) * 5 * 2 * kTfB;
-    for (int x = tid; x < 5 * 2 * kTfB; x += kTfB * kTfWaves) {
-        const int c = x / (2 * kTfB), slot = x % (2 * kTfB);
-        const bool jr = slot >= kTfB;
-        const int q = jr ? slot - kTfB : slot;
-        double v = 0.0;
-        if (c < 4) {
-            for (int u = 0; u < kTfWaves; u++) v += jr ? acc[u][c][q] : own[u][c][q];
-        } else {
-            int k = 0;
-            for (int u = 0; u < kTfWaves; u++) k += met[u][slot];
-            v = k;
-        }
-        o[x] = v;
+    // The last work-group out leaves the queue empty for the next launch.
+    if (queued && tid == 0 &&
+        __hip_atomic_fetch_add(queue + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+            gridDim.x - 1) {
+        reset_counter(queue);
+        reset_counter(queue + 1);
     }
 }
 
@@ -573,32 +599,37 @@ long tf_part_doubles(int np) {
     return nb * (nb + 1) / 2 * 5 * 2 * kTfB;
 }
 
-void launch_tf_rows(hipStream_t s, const PDev& p, int i_lo, int i_hi) {
-    const int nb = tf_blocks(p.np);
-    if (p.np == 0 || i_hi <= i_lo) return;
-    const dim3 g(nb, i_hi - i_lo);
-    if (p.n_typ <= kTfLdsTypes)
-        MAZE_LAUNCH(k_tf_tiles<true>, g, dim3(kTfB * kTfWaves), 0, s, p.np, p.n_typ, p.L,
-                    1.0 / p.L, p.r_cut, p.pos, p.types, p.table, p.tpart, i_lo);
-    else
-        MAZE_LAUNCH(k_tf_tiles<false>, g, dim3(kTfB * kTfWaves), 0, s, p.np, p.n_typ, p.L,
-                    1.0 / p.L, p.r_cut, p.pos, p.types, p.table, p.tpart, i_lo);
+// Whether the pair kernel leaves room for a solve that it runs beside and that
+// outlasts it.  With a work-group per block pair, the large tiles of the multigrid
+// levels find no CU with enough free registers and LDS until the last pairs are out
+// (1.03 ms for a 13 us kernel at 256^3); two work-groups per CU that take pairs from a
+// queue cost the pair kernel itself a quarter.  A 40-step run of 32768 ions on 256^3
+// takes 156 ms (166 with all work-groups at once, 162 with three per CU), of 21952 on
+// 224^3 256 (255), of 13824 on 192^3 152 (152).  Not where the pairs outlast the solve
+// (32768 ions on 128^3: 110 against 104 ms), where they are few (8000 ions: 118.3
+// against 117.2), or on grids whose CG solves take all CUs for themselves.
+bool tf_beside(int n, int np) {
+    const int nb = tf_blocks(np), items = tf_item(nb, nb, nb);
+    return (long)n * n * n >= 64L * items && items >= 64 * kTfCus &&
+           !cg_onchip2_fits(grid_dims_for(n));
 }
 
-void launch_tf_finish(hipStream_t s, const PDev& p, PScalars* ps, Reduce red) {
+void launch_tf(hipStream_t s, const PDev& p, PScalars* ps, Reduce red) {
     if (p.np == 0) {
         launch_sum_scaled(s, 0, 0.5, p.eion, &ps->pe_tf, red);
         return;
     }
-    const int nb = tf_blocks(p.np);
-    MAZE_LAUNCH(k_tf_fold, dim3(nb), dim3(kTfB * kFoldGroups), 0, s, p.np, nb, p.tpart,
-                       p.fn, p.eion, p.counts);
+    const int nb = tf_blocks(p.np), items = tf_item(nb, nb, nb);
+    const dim3 g(tf_beside(p.n, p.np) ? 2 * kTfCus : items), b(kTfB * kTfWaves);
+    if (p.n_typ <= kTfLdsTypes)
+        MAZE_LAUNCH(k_tf_tiles<true>, g, b, 0, s, p.np, p.n_typ, p.L, 1.0 / p.L, p.r_cut, p.pos,
+                    p.types, p.table, p.tpart, ps->tf_queue);
+    else
+        MAZE_LAUNCH(k_tf_tiles<false>, g, b, 0, s, p.np, p.n_typ, p.L, 1.0 / p.L, p.r_cut, p.pos,
+                    p.types, p.table, p.tpart, ps->tf_queue);
+    MAZE_LAUNCH(k_tf_fold, dim3(nb), dim3(kTfB * kFoldGroups), 0, s, p.np, nb, p.tpart, p.fn,
+                p.eion, p.counts);
     launch_sum_scaled(s, p.np, 0.5, p.eion, &ps->pe_tf, red);
-}
-
-void launch_tf(hipStream_t s, const PDev& p, PScalars* ps, Reduce red) {
-    launch_tf_rows(s, p, 0, tf_blocks(p.np));
-    launch_tf_finish(s, p, ps, red);
 }
 
 // F_tot = 0 + 1 F_elec + 1 F_noel [+ 1 F_db + 1 F_ib + 1 F_np]

@@ -43,6 +43,7 @@ struct PScalars {
     double typesum[3 * 16];
     int pb_flag;       // set by the PB map kernel when a tile overflows
     unsigned int epoch;  // charge spreads completed (tags the node lists)
+    unsigned int tf_queue[2];  // pair kernel: block pairs taken, work-groups done
 };
 
 void launch_cic_base(hipStream_t s, const PDev& p);
@@ -60,11 +61,7 @@ void launch_force_fd_kick(hipStream_t s, const PDev& p, const double* phi, doubl
                           const int* gate = nullptr);
 long tf_part_doubles(int np);
 void launch_tf(hipStream_t s, const PDev& p, PScalars* ps, Reduce red);
-// The same in pieces: the 64-ion block pairs (I, J >= I) of rows I in [i_lo, i_hi),
-// then the per-ion fold and the energy (after every row has run).
-int tf_blocks(int np);
-void launch_tf_rows(hipStream_t s, const PDev& p, int i_lo, int i_hi);
-void launch_tf_finish(hipStream_t s, const PDev& p, PScalars* ps, Reduce red);
+bool tf_beside(int n, int np);
 // F_tot = F_elec + F_noel (+ the PB boundary forces fdb, fib, fnp when given).
 void launch_force_total(hipStream_t s, const PDev& p, const double* fdb = nullptr,
                         const double* fib = nullptr, const double* fnp = nullptr);

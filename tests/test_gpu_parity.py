@@ -810,6 +810,28 @@ def test_tf_blocks_match_oracle(hip, oracle, oracle_raw, n_p, n_typ):
     assert abs(v - vo) <= u * vm.sum()
 
 
+# Block pairs from a queue (the larger grid) and a work-group each: the same bits, and
+# an emptied queue each time.
+@pytest.mark.parametrize("n_p", [11649, 13824])
+def test_tf_queue_equals_grid(hip, n_p):
+    s = W.nacl_system(13824, 164, seed=3)
+    s = dataclasses.replace(s, **{k: getattr(s, k)[:n_p] for k in ("types", "pos", "vel", "mass",
+                                                                   "charges")})
+    out = []
+    for n in (100, 164, 164):
+        driver.initialize(hip, dataclasses.replace(s, n_grid=n), driver.RunConfig(tol=1.0))
+        for _ in range(2):
+            v = hip.solver_compute_forces_noel()
+            f, cnt = np.zeros((n_p, 3)), np.zeros(n_p, dtype=np.int32)
+            hip.get_fcs_noel(f)
+            hip.get_tf_neighbor_counts(cnt)
+            out.append((v, f, cnt))
+        hip.solver_finalize()
+    assert np.abs(out[0][1]).max() > 0
+    for v, f, cnt in out[1:]:
+        assert v == out[0][0] and np.array_equal(f, out[0][1]) and np.array_equal(cnt, out[0][2])
+
+
 # ---- Poisson-Boltzmann boundary from ion radii -------------------------------------
 
 PB_RADII_SYSTEMS = {
