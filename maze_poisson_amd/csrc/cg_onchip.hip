@@ -2,8 +2,10 @@
 //
 // The sweeps of the single-reduction CG iteration (k_cg1_dir, k_cg1_update,
 // grid_kernels.hip) move 64 B per point and iteration through the memory
-// hierarchy and pay two kernel boundaries, although x, r, p and A p of a 128^3
-// grid (67 MB) fit the chip's registers and LDS (128 + 40 MB).  Here one
+// hierarchy and pay two kernel boundaries (32 us at 128^3, 14 us at 64^3 and
+// 32^3), although x, r, p and A p of a 128^3 grid (67 MB) fit the chip's
+// registers and LDS (128 + 40 MB).  9.7, 5.0 and 3.7 us here, of which the
+// exchange of the sums takes 2.3.  Here one
 // work-group per CU keeps its share of the grid for the whole solve: x, r and
 // A p in registers, p (with its in-plane halo) and the halo's r in LDS.  Per
 // iteration it exchanges one set of sums with all work-groups and the halo of

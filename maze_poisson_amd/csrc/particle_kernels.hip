@@ -353,8 +353,9 @@ void launch_force_fd_kick(hipStream_t s, const PDev& p, const double* phi, doubl
 // coefficients formed once, LDS adds without a return, pairs counted in ballots, no
 // bounds checks in full blocks.  Blocks whose extents lie further apart than the
 // cutoff are skipped.  Fewer work-groups than block pairs take theirs from a queue
-// (tf_beside).  32768 ions 1.94 ms (2.14 with the library's root, division and
-// rounding), 4096 50 us (56), 216 10.9 us (12.6); the sums keep their order and bits.
+// (tf_beside).  32768 ions 1.94 ms, or 2.4 beside the solve (2.14 with the library's
+// root, division and rounding), 4096 41 us (56; 50 with the launch grid's lower half
+// empty), 216 10.9 us (12.6); the sums keep their order and bits.
 constexpr int kTfB = 64;
 constexpr int kTfWaves = 4;
 constexpr int kTfCus = 256;
