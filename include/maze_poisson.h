@@ -279,6 +279,9 @@ int maze_test_conj_grad_pb(const double *b, double *x, double tol, int n, const 
 int maze_test_conj_grad_form(const double *b, double *x, double tol, int n, const double *eps_x,
                              const double *eps_y, const double *eps_z, const double *k2,
                              int reductions, int onchip);
+/* The set of exchange words (of as many as there are) that the one-launch form uses for
+ * its exchange of sums number `exchange`. */
+int maze_test_exchange_set(unsigned int exchange);
 /* The direct Poisson solve (n even, at most 256; x without the constant mode);
  * returns n, or -1 for another n. */
 int maze_test_spectral(const double *b, double *x, int n);

@@ -411,6 +411,8 @@ int maze_test_conj_grad_pb(const double* b, double* x, double tol, int n, const 
     return maze_test_conj_grad_form(b, x, tol, n, ex, ey, ez, k2, 1, 0);
 }
 
+int maze_test_exchange_set(unsigned int exchange) { return maze::exchange_set(exchange); }
+
 int maze_test_spectral(const double* b, double* x, int n) {
     if (!maze::spectral_ok(n)) return -1;
     Sim* s = scratch_sim(n);

@@ -26,9 +26,9 @@
 // slots, 2.7 and 3.2 us with several slots to a line).  A p values that
 // neighbours need are stored device-wide before (vmcnt(0), work-group barrier)
 // the work-group's sums are; a work-group that sees a neighbour's epoch may
-// read them, while the sums are on their way.  They alternate between two
-// buffers: the next but one exchange's values overwrite them, by when every
-// work-group has published the next exchange and so has read them.
+// read them, while the sums are on their way.  Values and words alternate between
+// two buffers: the next but one exchange overwrites them, by when every work-group
+// has published the next exchange and so has seen this one (exchange_set).
 //
 // Every wait ends: a poll that lasts longer than kWaitTicks marks the solve as
 // abandoned (kPoison in ctl), which every other wait sees.  x is written only
@@ -53,12 +53,14 @@ constexpr int kMaxGroups = kMaxWg / kWave;
 constexpr int kVals = kCg1Sums + 1;  // the sums and max|r|
 constexpr int kLine = 16;            // words per 128-byte line
 constexpr int kHalo = 8;             // in-plane halo entries per thread, at most
+constexpr int kSlot = kExchangeSets * kLine;  // words per work-group or group: a line per set
+constexpr int kSumsAt = kSlot * kMaxWg;       // the groups' slots
 
 struct OnchipArgs {
     GridDims d;
     int groups, nwg;  // work-groups per slab, all of them
-    u64* slots;       // per work-group kLine words: a pair per value
-    u64* sums;        // per group of 64 work-groups the same
+    u64* words;       // a slot per work-group, per line a pair per value; at kSumsAt the
+                      // same per group of 64 work-groups
     double *h0, *h1;  // A p values for the neighbours, by grid index, alternating
     unsigned int* ctl;
     unsigned int epoch;
@@ -138,7 +140,7 @@ __device__ __forceinline__ bool poll_slots(const u64* slots, int at, int cnt, un
         u64 a[8], b[8];
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            const u64* w = slots + kLine * min(at + 8 * i, cnt - 1);
+            const u64* w = slots + kSlot * min(at + 8 * i, cnt - 1);
             a[i] = word(w);
             b[i] = word(w + 1);
         }
@@ -312,6 +314,8 @@ __global__ __launch_bounds__(kThreads) void k_cg_onchip(OnchipArgs A, PBCoef pb,
             }
         }
         e++;
+        u64* const slots = A.words + exchange_set(e) * kLine;
+        u64* const sums = slots + kSumsAt;
         // The tiles' sums and their pair's, published once the work-group's
         // A p values have arrived.
 #pragma unroll
@@ -328,7 +332,7 @@ __global__ __launch_bounds__(kThreads) void k_cg_onchip(OnchipArgs A, PBCoef pb,
         const int val = lane & 7, sub = lane / 8;  // a lane's value and place among 8 slots
         if (wv == 0) {
             if (lane < kVals)
-                put(A.slots + kLine * blockIdx.x + 2 * lane,
+                put(slots + kSlot * blockIdx.x + 2 * lane,
                     lane < kCg1Sums ? cg1_pair(shw[lane], shw[lane] + 4)
                                     : cg1_pair_max(shw[lane], shw[lane] + 4),
                     e);
@@ -344,7 +348,7 @@ __global__ __launch_bounds__(kThreads) void k_cg_onchip(OnchipArgs A, PBCoef pb,
             const int slot = s_ * A.groups + (q < 2 ? g0 : p / nt);
             if (q < 6) {
                 double v[1];
-                ok = poll<1>(A.slots + kLine * slot, 0, e, A.ctl, v);
+                ok = poll<1>(slots + kSlot * slot, 0, e, A.ctl, v);
             }
         } else if (wv == 2) {
             // Group g of 64 slots is folded by work-group g.
@@ -352,9 +356,9 @@ __global__ __launch_bounds__(kThreads) void k_cg_onchip(OnchipArgs A, PBCoef pb,
             for (int g = blockIdx.x; g < J; g += A.nwg) {
                 const int at = vopaque(g * kWave + sub);
                 double v[8];
-                ok = poll_slots(A.slots + 2 * (val < kVals ? val : 0), at, A.nwg, e, A.ctl, v);
+                ok = poll_slots(slots + 2 * (val < kVals ? val : 0), at, A.nwg, e, A.ctl, v);
                 const double f = cg1_fold(v, val == kCg1Sums);
-                if (sub == 0 && val < kVals) put(A.sums + kLine * g + 2 * val, f, e);
+                if (sub == 0 && val < kVals) put(sums + kSlot * g + 2 * val, f, e);
             }
         }
         if (!ok) bad = 1;
@@ -376,7 +380,7 @@ __global__ __launch_bounds__(kThreads) void k_cg_onchip(OnchipArgs A, PBCoef pb,
         if (wv == 0) {
             const int g = min(sub, J - 1);
             double v[1];
-            ok = poll<1>(A.sums + kLine * g + 2 * (val < kVals ? val : 0), 0, e, A.ctl, v);
+            ok = poll<1>(sums + kSlot * g + 2 * (val < kVals ? val : 0), 0, e, A.ctl, v);
             double S[kVals];
 #pragma unroll
             for (int c = 0; c < kVals; c++) {
@@ -491,8 +495,8 @@ __global__ __launch_bounds__(kThreads) void k_cg_onchip(OnchipArgs A, PBCoef pb,
 struct Onchip2Args {
     GridDims d;
     int T, groups, nwg;  // tiles per work-group, work-groups per slab, all of them
-    u64* slots;          // a line per work-group: a pair per tile, then max|r|
-    u64* sums;           // a line per group of 64 slots: sum, max
+    u64* words;          // a slot per work-group, per line a pair per tile, then max|r|; at
+                         // kSumsAt per group of 64 slots the sum and max
     double* h;           // r values for the neighbours, by grid index
     unsigned int* ctl;
     unsigned int epoch;
@@ -585,6 +589,7 @@ __global__ __launch_bounds__(NT) void k_cg_onchip2(Onchip2Args A, PBCoef pb, dou
     }
     __syncthreads();
 
+    auto slots = [&]() { return A.words + exchange_set(e) * kLine; };
     // This work-group's tile sums (and max) to its line, as block_sum forms them.
     auto publish = [&](double s, double m, bool with_max) {
         s = wave_sum_rows(s);
@@ -598,12 +603,12 @@ __global__ __launch_bounds__(NT) void k_cg_onchip2(Onchip2Args A, PBCoef pb, dou
         if (wv == 0 && lane < tiles) {
             double v = 0.0;
             for (int w = 0; w < kBlock / kWave; w++) v += shw[0][lane * (kBlock / kWave) + w];
-            put(A.slots + kLine * blockIdx.x + 2 * lane, v, e);
+            put(slots() + kSlot * blockIdx.x + 2 * lane, v, e);
         }
         if (with_max && wv == 0 && lane == kMaxTiles) {
             double v = 0.0;
             for (int w = 0; w < nt / kWave; w++) v = fmax(v, shw[1][w]);
-            put(A.slots + kLine * blockIdx.x + 2 * kMaxTiles, v, e);
+            put(slots() + kSlot * blockIdx.x + 2 * kMaxTiles, v, e);
         }
     };
     // Lanes of group g hold the partials 64 g + lane + 256 u in the sweeps' order
@@ -616,10 +621,10 @@ __global__ __launch_bounds__(NT) void k_cg_onchip2(Onchip2Args A, PBCoef pb, dou
             const int xs = g * kWave + lane + u * kBlock;
             const int tile = xcd_tile(min(xs, nb - 1), nb);
             const int ts = tile / A.d.chunks, ch = tile - ts * A.d.chunks, gg = ch / A.T;
-            off[u] = xs < nb ? kLine * (ts * A.groups + gg) + 2 * (ch - gg * A.T) : -1;
+            off[u] = xs < nb ? kSlot * (ts * A.groups + gg) + 2 * (ch - gg * A.T) : -1;
         }
         const int wg = g * kWave + lane;
-        off[kFoldSlots / kBlock] = wg < A.nwg ? kLine * wg + 2 * kMaxTiles : -1;
+        off[kFoldSlots / kBlock] = wg < A.nwg ? kSlot * wg + 2 * kMaxTiles : -1;
     };
     int mine[kFoldSlots / kBlock + 1];
     offsets(blockIdx.x, mine);
@@ -631,9 +636,9 @@ __global__ __launch_bounds__(NT) void k_cg_onchip2(Onchip2Args A, PBCoef pb, dou
             if (g != (int)blockIdx.x) offsets(g, mine);
             double v[kFoldSlots / kBlock + 1];
             if (with_max) {
-                ok = poll_at<kFoldSlots / kBlock + 1>(A.slots, mine, e, A.ctl, v) && ok;
+                ok = poll_at<kFoldSlots / kBlock + 1>(slots(), mine, e, A.ctl, v) && ok;
             } else {
-                ok = poll_at<kFoldSlots / kBlock>(A.slots, mine, e, A.ctl, v) && ok;
+                ok = poll_at<kFoldSlots / kBlock>(slots(), mine, e, A.ctl, v) && ok;
                 v[kFoldSlots / kBlock] = 0.0;
             }
             double s = 0.0;
@@ -641,8 +646,8 @@ __global__ __launch_bounds__(NT) void k_cg_onchip2(Onchip2Args A, PBCoef pb, dou
             for (int u = 0; u < kFoldSlots / kBlock; u++) s += v[u];
             s = wave_sum_rows(s);
             const double m = wave_max_dpp(v[kFoldSlots / kBlock]);
-            if (lane == 0) put(A.sums + kLine * g, s, e);
-            if (with_max && lane == 1) put(A.sums + kLine * g + 2, m, e);
+            if (lane == 0) put(slots() + kSumsAt + kSlot * g, s, e);
+            if (with_max && lane == 1) put(slots() + kSumsAt + kSlot * g + 2, m, e);
         }
         if (A.nwg < kBlock / kWave) offsets(blockIdx.x, mine);
         return ok;
@@ -651,7 +656,7 @@ __global__ __launch_bounds__(NT) void k_cg_onchip2(Onchip2Args A, PBCoef pb, dou
     auto totals = [&](bool with_max, double& S, double& M) {
         const int g = min(lane / 8, kBlock / kWave - 1), c = with_max ? min(lane & 7, 1) : 0;
         double v[1];
-        const bool ok = poll<1>(A.sums + kLine * g + 2 * c, 0, e, A.ctl, v);
+        const bool ok = poll<1>(slots() + kSumsAt + kSlot * g + 2 * c, 0, e, A.ctl, v);
         S = M = 0.0;
 #pragma unroll
         for (int q = 0; q < kBlock / kWave; q++) {
@@ -748,7 +753,7 @@ __global__ __launch_bounds__(NT) void k_cg_onchip2(Onchip2Args A, PBCoef pb, dou
             const int slot = s_ * A.groups + (q < 2 ? g0 : p / nt);
             if (q < 6) {
                 double v[1];
-                ok = poll<1>(A.slots + kLine * slot, 0, e, A.ctl, v);
+                ok = poll<1>(slots() + kSlot * slot, 0, e, A.ctl, v);
             }
         }
         ok = fold_groups(true) && ok;
@@ -880,8 +885,7 @@ constexpr int kStreamStride = kThreads + 4;  // a plane in LDS: p, then the ends
 struct StreamArgs {
     GridDims d;
     int groups, slabs, nwg;  // work-groups per slab, slabs of work-groups, all of them
-    u64* slots;              // a line per work-group: up to four tiles' sums, max|r|, p ready
-    u64* sums;
+    u64* words;              // as Onchip2Args, per line: up to four tiles' sums, max|r|, p ready
     double* h;               // p on the edges, by grid index
     double* xs;              // x after the first update (x itself is written at the end)
     unsigned int* ctl;
@@ -946,6 +950,9 @@ __global__ __launch_bounds__(kThreads) void k_cg_stream(StreamArgs A, PBCoef pb,
         if (act && u < ni) lds[u * LP + idx] = R[u] * cr;
     }
 
+    // The words of an iteration's first and second exchange; those that tell that p is
+    // ready are written once an iteration, with both exchanges between, and need one set.
+    auto slots = [&](bool second) { return A.words + exchange_set(second ? 1 : 0) * kLine; };
     // Tile sums (of two slabs' parts) and max to this work-group's line.
     auto publish = [&](double s0, double s1, double m, bool with_max) {
         s0 = wave_sum_rows(s0);
@@ -961,12 +968,12 @@ __global__ __launch_bounds__(kThreads) void k_cg_stream(StreamArgs A, PBCoef pb,
             const double* w = &shw[lane >> 1][(lane & 1) * (kBlock / kWave)];
             double v = 0.0;
             for (int q = 0; q < kBlock / kWave; q++) v += w[q];
-            put(A.slots + kLine * blockIdx.x + 2 * lane, v, e);
+            put(slots(with_max) + kSlot * blockIdx.x + 2 * lane, v, e);
         }
         if (with_max && wv == 0 && lane == kMaxTiles) {
             double v = 0.0;
             for (int w = 0; w < NW; w++) v = fmax(v, shw[2][w]);
-            put(A.slots + kLine * blockIdx.x + 2 * kMaxTiles, v, e);
+            put(slots(with_max) + kSlot * blockIdx.x + 2 * kMaxTiles, v, e);
         }
     };
     // As in k_cg_onchip2; tile (slab, chunk) is part 2 (slab past the last
@@ -978,10 +985,10 @@ __global__ __launch_bounds__(kThreads) void k_cg_stream(StreamArgs A, PBCoef pb,
             const int tile = xcd_tile(min(xs, nb - 1), nb);
             const int ts = tile / A.d.chunks, ch = tile - ts * A.d.chunks;
             const int ws = min(ts, A.slabs - 1);
-            off[u] = xs < nb ? kLine * (ws * A.groups + ch / 2) + 2 * (2 * (ts - ws) + (ch & 1)) : -1;
+            off[u] = xs < nb ? kSlot * (ws * A.groups + ch / 2) + 2 * (2 * (ts - ws) + (ch & 1)) : -1;
         }
         const int wg = g * kWave + lane;
-        off[kFoldSlots / kBlock] = wg < A.nwg ? kLine * wg + 2 * kMaxTiles : -1;
+        off[kFoldSlots / kBlock] = wg < A.nwg ? kSlot * wg + 2 * kMaxTiles : -1;
     };
     int mine[kFoldSlots / kBlock + 1];
     offsets(blockIdx.x, mine);
@@ -990,9 +997,9 @@ __global__ __launch_bounds__(kThreads) void k_cg_stream(StreamArgs A, PBCoef pb,
         double v[kFoldSlots / kBlock + 1];
         bool ok;
         if (with_max) {
-            ok = poll_at<kFoldSlots / kBlock + 1>(A.slots, mine, e, A.ctl, v);
+            ok = poll_at<kFoldSlots / kBlock + 1>(slots(with_max), mine, e, A.ctl, v);
         } else {
-            ok = poll_at<kFoldSlots / kBlock>(A.slots, mine, e, A.ctl, v);
+            ok = poll_at<kFoldSlots / kBlock>(slots(with_max), mine, e, A.ctl, v);
             v[kFoldSlots / kBlock] = 0.0;
         }
         double s = 0.0;
@@ -1000,14 +1007,14 @@ __global__ __launch_bounds__(kThreads) void k_cg_stream(StreamArgs A, PBCoef pb,
         for (int u = 0; u < kFoldSlots / kBlock; u++) s += v[u];
         s = wave_sum_rows(s);
         const double m = wave_max_dpp(v[kFoldSlots / kBlock]);
-        if (lane == 0) put(A.sums + kLine * blockIdx.x, s, e);
-        if (with_max && lane == 1) put(A.sums + kLine * blockIdx.x + 2, m, e);
+        if (lane == 0) put(slots(with_max) + kSumsAt + kSlot * blockIdx.x, s, e);
+        if (with_max && lane == 1) put(slots(with_max) + kSumsAt + kSlot * blockIdx.x + 2, m, e);
         return ok;
     };
     auto totals = [&](bool with_max, double& S, double& M) {
         const int g = min(lane / 8, kBlock / kWave - 1), c = with_max ? min(lane & 7, 1) : 0;
         double v[1];
-        const bool ok = poll<1>(A.sums + kLine * g + 2 * c, 0, e, A.ctl, v);
+        const bool ok = poll<1>(slots(with_max) + kSumsAt + kSlot * g + 2 * c, 0, e, A.ctl, v);
         S = M = 0.0;
 #pragma unroll
         for (int q = 0; q < kBlock / kWave; q++) {
@@ -1030,7 +1037,7 @@ __global__ __launch_bounds__(kThreads) void k_cg_stream(StreamArgs A, PBCoef pb,
         __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         bool ok = true;
-        if (wv == 0 && lane == 0) put(A.slots + kLine * blockIdx.x + kReadyWord, 0.0, e);
+        if (wv == 0 && lane == 0) put(A.words + kSlot * blockIdx.x + kReadyWord, 0.0, e);
         if (wv == 1) {
             const int q = vopaque(lane);
             const int p = wrap(q == 2 ? base - n : q == 3 ? base - 1 : q == 4 ? base + cnt
@@ -1040,7 +1047,7 @@ __global__ __launch_bounds__(kThreads) void k_cg_stream(StreamArgs A, PBCoef pb,
             const int slot = s_ * A.groups + (q < 2 ? g0 : p / nt);
             if (q < 6) {
                 double v[1];
-                ok = poll<1>(A.slots + kLine * slot + kReadyWord, 0, e, A.ctl, v);
+                ok = poll<1>(A.words + kSlot * slot + kReadyWord, 0, e, A.ctl, v);
             }
         }
         // Waves 2 to 4: the ends of cut rows (nothing that is used where a row starts
@@ -1051,7 +1058,7 @@ __global__ __launch_bounds__(kThreads) void k_cg_stream(StreamArgs A, PBCoef pb,
             const int p = q == 0 ? max(base - 1, 0) : q == 1 ? first : q == 2 ? min(base + cnt, n2 - 1)
                                                                               : last;
             double v[1];
-            ok = poll<1>(A.slots + kLine * (sl * A.groups + g) + kReadyWord, 0, e, A.ctl, v);
+            ok = poll<1>(A.words + kSlot * (sl * A.groups + g) + kReadyWord, 0, e, A.ctl, v);
             lds[u * LP + nt + q] = load_partial(A.h, (i0 + u) * n2 + p);
         }
         if (!ok) bad = 1;
@@ -1377,7 +1384,7 @@ bool cg_onchip_fits(const GridDims& d) {
     return share_fits(d) && groups_of(d) * d.slabs <= compute_units();
 }
 
-long cg_onchip_words() { return (long)kLine * (kMaxWg + kMaxGroups); }
+long cg_onchip_words() { return kSlot * (kMaxWg + kMaxGroups); }
 
 void launch_cg_onchip(hipStream_t s, const GridDims& d, const PBCoef& pb, double* x, double* r,
                       double* h0, double* h1, CGState* st, const CgOnchip& w) {
@@ -1385,8 +1392,7 @@ void launch_cg_onchip(hipStream_t s, const GridDims& d, const PBCoef& pb, double
     a.d = d;
     a.groups = groups_of(d);
     a.nwg = a.groups * d.slabs;
-    a.slots = w.words;
-    a.sums = w.words + (long)kLine * kMaxWg;
+    a.words = w.words;
     a.h0 = h0;
     a.h1 = h1;
     a.ctl = w.ctl;
@@ -1411,8 +1417,7 @@ void launch_cg_onchip2(hipStream_t s, const GridDims& d, const PBCoef& pb, doubl
         b.groups = groups_of(d);
         b.slabs = stream_slabs(d, compute_units());
         b.nwg = b.groups * b.slabs;
-        b.slots = w.words;
-        b.sums = w.words + (long)kLine * kMaxWg;
+        b.words = w.words;
         b.h = h;
         b.xs = xs;
         b.ctl = w.ctl;
@@ -1424,8 +1429,7 @@ void launch_cg_onchip2(hipStream_t s, const GridDims& d, const PBCoef& pb, doubl
     }
     a.groups = (d.chunks + a.T - 1) / a.T;
     a.nwg = a.groups * d.slabs;
-    a.slots = w.words;
-    a.sums = w.words + (long)kLine * kMaxWg;
+    a.words = w.words;
     a.h = h;
     a.ctl = w.ctl;
     a.epoch = w.epoch;

@@ -134,6 +134,13 @@ void launch_cg1_update(hipStream_t s, const GridDims& d, const PBCoef& pb, const
 // h0, h1: scratch grids; words: cg_onchip_words() of them, zeroed once; epoch:
 // advances by more than the iterations + 2 per launch, words zeroed again
 // before it wraps.
+// A launch's exchanges of sums alternate between two sets of words: work-groups that
+// have seen an exchange's sums publish the next one while others still look for this
+// one's, and are held up at the next but one, which needs everyone's next.
+constexpr int kExchangeSets = 2;
+__host__ __device__ constexpr int exchange_set(unsigned int exchange) {
+    return (int)(exchange % kExchangeSets);
+}
 struct CgOnchip {
     unsigned long long* words;
     unsigned int* ctl;

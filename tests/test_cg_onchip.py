@@ -119,3 +119,74 @@ def test_abandoned_launch_falls_back(hip_raw, n, reductions):
     assert _solve(hip_raw, b, xs, tol, n, reductions, 0) >= 0
     assert _solve(hip_raw, b, xo, tol, n, reductions, 2) == -3
     assert np.array_equal(xo, xs)
+
+
+# ---- the exchange of sums, as a model ----------------------------------------------
+# Every work-group puts its slot of an exchange and waits for the totals; the first
+# work-group of a group of slots folds them into the group's sum; where the halo is
+# exchanged too, another wave waits for the neighbours' slots.  A wait is for the exact
+# epoch, so a word must not move on before everyone who looks for it has seen it.
+WGS, PER_GROUP, EXCHANGES = 6, 2, 8
+
+
+def _waves(w, form, exchange_set):
+    """The waves of work-group w as lists of ("put" | "wait", words, epoch) and "meet"."""
+    groups = WGS // PER_GROUP
+    w0, w1, w2 = [], [], []
+    for e in range(1, EXCHANGES + 1):
+        s = exchange_set(e)
+        halo = form == 1 or e % 2 == 0
+        w0.append(("put", [("slot", s, w)], e))
+        if halo:
+            w1.append(("wait", [("slot", s, (w + d) % WGS) for d in (1, WGS - 1)], e))
+        if w < groups:
+            w2.append(("wait", [("slot", s, PER_GROUP * w + q) for q in range(PER_GROUP)], e))
+            w2.append(("put", [("sum", s, w)], e))
+        totals = ("wait", [("sum", s, g) for g in range(groups)], e)
+        if halo:  # the totals are taken once the neighbours' values are there
+            for x in (w0, w1, w2):
+                x.append("meet")
+        w0.append(totals)
+        for x in (w0, w1, w2):
+            x.append("meet")
+    return [w0, w1, w2]
+
+
+def _lost_waits(form, exchange_set):
+    """Waits that never end if their wave is held up until all others are stuck."""
+    progs = {(w, v): p for w in range(WGS) for v, p in enumerate(_waves(w, form, exchange_set))}
+    lost = []
+    for victim, prog in progs.items():
+        for stop in [i for i, op in enumerate(prog) if op != "meet" and op[0] == "wait"]:
+            at, mem, moved = dict.fromkeys(progs, 0), {}, True
+            while moved:
+                moved = False
+                for a, p in progs.items():
+                    if at[a] == len(p) or (a == victim and at[a] == stop):
+                        continue
+                    op = p[at[a]]
+                    if op == "meet":  # all three waves of a work-group have come to it
+                        if all(at[b] < len(progs[b]) and progs[b][at[b]] == "meet" and
+                               progs[b][:at[b]].count("meet") == p[:at[a]].count("meet")
+                               for b in progs if b[0] == a[0]):
+                            for b in progs:
+                                at[b] += b[0] == a[0]
+                            moved = True
+                    elif op[0] == "put":
+                        mem.update({x: op[2] for x in op[1]})
+                        at[a] += 1
+                        moved = True
+                    elif all(mem.get(x) == op[2] for x in op[1]):
+                        at[a] += 1
+                        moved = True
+            if at[victim] == stop and any(mem.get(x) != prog[stop][2] for x in prog[stop][1]):
+                lost.append((victim, prog[stop]))
+    return lost
+
+
+@pytest.mark.parametrize("form", [1, 2])
+def test_no_exchange_is_missed(hip, form):
+    f = hip.lib.maze_test_exchange_set
+    f.restype, f.argtypes = ctypes.c_int, [ctypes.c_uint]
+    assert _lost_waits(form, f) == []
+    assert _lost_waits(form, lambda e: 0)  # one set of words: a late look finds them gone
