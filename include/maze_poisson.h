@@ -275,10 +275,14 @@ int maze_test_conj_grad_pb(const double *b, double *x, double tol, int n, const 
 /* The same solves (ex == NULL: Poisson) with one or two reductions per
  * iteration, as sweeps (onchip 0) or as one launch with the CG vectors on the
  * chip (bit-identical; -2 if the grid does not fit it, -3 if the launch was
- * abandoned and the sweeps ran; onchip 2: it starts abandoned). */
+ * abandoned and the sweeps ran; onchip 2: it starts abandoned; onchip 3: the epochs
+ * start anew with it, -4 if they do not). */
 int maze_test_conj_grad_form(const double *b, double *x, double tol, int n, const double *eps_x,
                              const double *eps_y, const double *eps_z, const double *k2,
                              int reductions, int onchip);
+/* The epoch that follows a launch from `epoch` that may have used `used` of them, for one
+ * that may use `span`; 0: they start anew. */
+unsigned int maze_test_next_epoch(unsigned int epoch, unsigned int used, unsigned int span);
 /* The set of exchange words (of as many as there are) that the one-launch form uses for
  * its exchange of sums number `exchange`. */
 int maze_test_exchange_set(unsigned int exchange);

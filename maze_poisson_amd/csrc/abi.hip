@@ -388,6 +388,12 @@ int maze_test_conj_grad_form(const double* b, double* x, double tol, int n, cons
         MAZE_HIP(hipMemcpy(s->sigma, b, s->G * sizeof(double), hipMemcpyHostToDevice));
         MAZE_HIP(hipMemcpy(s->y, x, s->G * sizeof(double), hipMemcpyHostToDevice));
         int pred = 32;
+        if (onchip == 3) {  // after a solve with the last epochs there are
+            s->onchip_next(s->cg_two() ? s->dims : s->cgd, n * n, s->cg_two());
+            s->onchip_w.epoch = 0xffffffffu - 2 * s->onchip_span;
+            s->cg_solve(s->cg_run(s->y, s->sigma, pred + 1, &pred));
+            MAZE_HIP(hipMemcpy(s->y, x, s->G * sizeof(double), hipMemcpyHostToDevice));
+        }
         if (onchip == 2) {
             s->onchip_next(s->cg_two() ? s->dims : s->cgd, n * n, s->cg_two());
             const unsigned int given_up = 1u << 30;
@@ -397,6 +403,7 @@ int maze_test_conj_grad_form(const double* b, double* x, double tol, int n, cons
         res = s->cg_solve(s->cg_run(s->y, s->sigma, pred + 1, &pred));
         MAZE_HIP(hipMemcpy(x, s->y, s->G * sizeof(double), hipMemcpyDeviceToHost));
         if (onchip && !s->onchip) res = -3;
+        if (onchip == 3 && s->onchip_w.epoch != 1u) res = -4;
     }
     delete s;
     return res;
@@ -409,6 +416,10 @@ int maze_test_conj_grad(const double* b, double* x, double tol, int n) {
 int maze_test_conj_grad_pb(const double* b, double* x, double tol, int n, const double* ex,
                            const double* ey, const double* ez, const double* k2) {
     return maze_test_conj_grad_form(b, x, tol, n, ex, ey, ez, k2, 1, 0);
+}
+
+unsigned int maze_test_next_epoch(unsigned int epoch, unsigned int used, unsigned int span) {
+    return maze::next_epoch(epoch, used, span);
 }
 
 int maze_test_exchange_set(unsigned int exchange) { return maze::exchange_set(exchange); }

@@ -146,6 +146,12 @@ struct CgOnchip {
     unsigned int* ctl;
     unsigned int epoch;
 };
+// The epoch of a launch that may use `span` epochs, after one from `epoch` that may have
+// used `used`; 0: the words are to be zeroed first, for epoch 1.
+inline unsigned int next_epoch(unsigned int epoch, unsigned int used, unsigned int span) {
+    const unsigned long long e = (unsigned long long)epoch + used;
+    return e + span <= 0xffffffffull ? (unsigned int)e : 0u;
+}
 // The launch shape of FP64 CG on an n^3 grid, in either form.
 GridDims cg_dims_for(int n);
 bool cg_onchip_fits(const GridDims& d);

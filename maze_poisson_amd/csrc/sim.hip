@@ -600,11 +600,12 @@ bool Sim::onchip_next(const GridDims& d, int limit, int two) {
         onchip_w.words = dalloc<unsigned long long>(words);
         onchip_w.ctl = dalloc<unsigned int>(1);
         onchip_w.epoch = 1u;
-    } else if (onchip_w.epoch > 0xffffffffu - 2u * span) {
-        launch_fill(stream, words, 0.0, reinterpret_cast<double*>(onchip_w.words));
-        onchip_w.epoch = 1u;
     } else {
-        onchip_w.epoch += onchip_span;
+        onchip_w.epoch = next_epoch(onchip_w.epoch, onchip_span, span);
+        if (!onchip_w.epoch) {
+            launch_fill(stream, words, 0.0, reinterpret_cast<double*>(onchip_w.words));
+            onchip_w.epoch = 1u;
+        }
     }
     onchip_span = span;
     return true;

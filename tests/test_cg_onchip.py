@@ -121,6 +121,35 @@ def test_abandoned_launch_falls_back(hip_raw, n, reductions):
     assert np.array_equal(xo, xs)
 
 
+# The first solve after the epochs have run out.
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,reductions", [(48, 1), (48, 2), (131, 2)])
+def test_epochs_start_anew(hip_raw, n, reductions):
+    b, x0 = _problem(n, 4)
+    tol = 1e-6 * np.abs(b).max()
+    xs, xo = x0.copy(), x0.copy()
+    i_s = _solve(hip_raw, b, xs, tol, n, reductions, 0)
+    assert _solve(hip_raw, b, xo, tol, n, reductions, 3) == i_s >= 0
+    assert np.array_equal(xo, xs)
+
+
+# No launch uses an epoch that may be in the words already, whatever the solves before
+# it: a long one (its span is its own cap) followed by short ones among them.
+def test_epochs_never_repeat(hip):
+    f = hip.lib.maze_test_next_epoch
+    f.restype, f.argtypes = ctypes.c_uint, [ctypes.c_uint] * 3
+    top = 2 ** 32 - 1
+    assert f(top - 100, 49158, 36) == 0
+    assert f(top - 72, 36, 36) == top - 36 and f(top - 71, 36, 36) == 0
+    g = np.random.default_rng(0)
+    epoch, used, low = 1, 6, 1
+    for span in (2 ** g.uniform(3, 31, 5000)).astype(np.uint64):
+        span = int(span)
+        e = f(epoch, used, span)
+        assert e == 0 or (e >= epoch + used >= low and e + span <= top)
+        epoch, used, low = (e, span, e) if e else (1, span, 1)
+
+
 # ---- the exchange of sums, as a model ----------------------------------------------
 # Every work-group puts its slot of an exchange and waits for the totals; the first
 # work-group of a group of slots folds them into the group's sum; where the halo is
