@@ -19,7 +19,7 @@ static Sim* g_sim = nullptr;
 static Sim& S() {
     if (!g_sim) {
         g_sim = new Sim();
-        g_sim->onchip = 1;
+        g_sim->onchip_enable();
     }
     return *g_sim;
 }
@@ -376,7 +376,7 @@ int maze_test_conj_grad_form(const double* b, double* x, double tol, int n, cons
                              const double* ey, const double* ez, const double* k2, int reductions,
                              int onchip) {
     Sim* s = scratch_sim(n);
-    s->onchip = onchip != 0;
+    if (onchip) s->onchip_enable();
     if (ex) {
         s->init_pb(0.0, 0.0);
         s->set_eps_k2(ex, ey, ez, k2);

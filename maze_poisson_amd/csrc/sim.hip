@@ -141,7 +141,8 @@ Sim::Sim(hipStream_t main, hipStream_t side_, HostBlock* block) {
     ps_host = &host->ps;
     pub_host = &host->pub;
     MAZE_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&pub_dev), pub_host, 0));
-    reserve(sizeof(double) * (7 + kCg1Sums) * (size_t)kMaxPartials + (64 << 10), 16);
+    reserve(sizeof(double) * ((7 + kCg1Sums) * (size_t)kMaxPartials + cg_onchip_words()) + (64 << 10),
+            16);
     red_side.psum = dalloc<double>(kMaxPartials);
     red_side.pmax = dalloc<double>(kMaxPartials);
     red_side.counter = dalloc<unsigned int>(kArrivalWords);
@@ -591,21 +592,22 @@ void Sim::cg_start() {
     launch_cg_init<double>(stream, cg.d, cg.pbc, cg.x, cg.b, cg.rbuf, st, red);
 }
 
+// The exchange words live as long as the replica, so they are allocated before the first
+// grid: a chunk is freed with its last allocation.
+void Sim::onchip_enable() {
+    onchip = 1;
+    onchip_w.words = dalloc<unsigned long long>(cg_onchip_words());
+    onchip_w.ctl = dalloc<unsigned int>(1);
+}
+
 bool Sim::onchip_next(const GridDims& d, int limit, int two) {
     // Per-kernel timing names the sweeps, so it runs them.
     if (!onchip || prof || !(two ? cg_onchip2_fits(d) : cg_onchip_fits(d))) return false;
-    const long words = cg_onchip_words();
     const unsigned int span = 3u * (unsigned int)limit + 6u;
-    if (!onchip_w.words) {
-        onchip_w.words = dalloc<unsigned long long>(words);
-        onchip_w.ctl = dalloc<unsigned int>(1);
+    onchip_w.epoch = next_epoch(onchip_w.epoch, onchip_span, span);
+    if (!onchip_w.epoch) {
+        launch_fill(stream, cg_onchip_words(), 0.0, reinterpret_cast<double*>(onchip_w.words));
         onchip_w.epoch = 1u;
-    } else {
-        onchip_w.epoch = next_epoch(onchip_w.epoch, onchip_span, span);
-        if (!onchip_w.epoch) {
-            launch_fill(stream, words, 0.0, reinterpret_cast<double*>(onchip_w.words));
-            onchip_w.epoch = 1u;
-        }
     }
     onchip_span = span;
     return true;

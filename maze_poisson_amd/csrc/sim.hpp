@@ -227,6 +227,7 @@ struct Sim {
     CgOnchip onchip_w{nullptr, nullptr, 1u};
     int onchip_void = 0;           // tests: the next launch starts abandoned
     unsigned int onchip_span = 0;  // epochs the last such solve may have used
+    void onchip_enable();  // right after the constructor
     // Whether the next solve on grid d goes on the chip (sets its exchange up).
     bool onchip_next(const GridDims& d, int limit, int two = 0);
     // FP64 CG runs with one reduction per iteration (Cg1) in the FP64 precisions.

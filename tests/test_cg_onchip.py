@@ -4,6 +4,8 @@ import ctypes
 import numpy as np
 import pytest
 
+from maze_poisson_amd import driver, workloads as W
+
 D = np.ctypeslib.ndpointer(dtype=np.float64, flags="C_CONTIGUOUS")
 FIT_MAX = 128  # the largest grid whose vectors fit
 
@@ -219,3 +221,19 @@ def test_no_exchange_is_missed(hip, form):
     f.restype, f.argtypes = ctypes.c_int, [ctypes.c_uint]
     assert _lost_waits(form, f) == []
     assert _lost_waits(form, lambda e: 0)  # one set of words: a late look finds them gone
+
+
+# A second grid without finalize gives the memory of the first one back.
+@pytest.mark.gpu
+def test_second_grid_frees_the_first(hip):
+    free_now, total = ctypes.c_size_t(), ctypes.c_size_t()
+    small, large = W.nacl_system(216, 32, seed=1), W.nacl_system(216, 128, seed=1)
+    free = []
+    for systems in ([small], [large, small]):
+        for s in systems:
+            driver.initialize(hip, s, driver.RunConfig(tol=W.poisson_tol(s)))
+            driver.bootstrap(hip)
+        assert hip.lib.hipMemGetInfo(ctypes.byref(free_now), ctypes.byref(total)) == 0
+        free.append(free_now.value)
+        hip.solver_finalize()
+    assert free[0] - free[1] < 16 << 20  # the first grid's arrays take 150 MB
