@@ -260,6 +260,11 @@ void maze_prof_enable(int on);
 void maze_prof_reset(void);
 int maze_prof_get(const char *name, double *total_ms, long *count);
 int maze_grid_blocks(void);
+/* FP64 CG solves of up to 128^3 (and the cold ones of the mixed modes at some larger
+ * sizes) run in one launch that needs the whole GPU.  One that waits for it in vain,
+ * 0.2 s, is run again in another form (the same result), as are the next 256 or more;
+ * stderr tells of the first.  How many since solver_initialize: */
+long maze_onchip_abandoned(void);
 /* One launch of the plain copy kernel over n doubles (reads and writes 8n
  * bytes): the calibration reference for hardware byte counters. */
 void maze_calib_copy(long n_doubles);
@@ -280,6 +285,9 @@ int maze_test_conj_grad_pb(const double *b, double *x, double tol, int n, const 
 int maze_test_conj_grad_form(const double *b, double *x, double tol, int n, const double *eps_x,
                              const double *eps_y, const double *eps_z, const double *k2,
                              int reductions, int onchip);
+/* `count` solves of b in turn, the first starting abandoned; on_chip[k]: whether solve k
+ * ran in one launch.  Returns how many were abandoned. */
+int maze_test_onchip_pause(const double *b, double tol, int n, int count, int *on_chip);
 /* The epoch that follows a launch from `epoch` that may have used `used` of them, for one
  * that may use `span`; 0: they start anew. */
 unsigned int maze_test_next_epoch(unsigned int epoch, unsigned int used, unsigned int span);

@@ -290,6 +290,8 @@ int maze_prof_get(const char* name, double* total_ms, long* count) {
     return -1;
 }
 
+long maze_onchip_abandoned() { return S().onchip_abandoned; }
+
 int maze_grid_blocks() { return S().dims.blocks; }
 
 // One launch of the plain copy kernel over n_doubles doubles (read n*8 bytes,
@@ -402,7 +404,7 @@ int maze_test_conj_grad_form(const double* b, double* x, double tol, int n, cons
         }
         res = s->cg_solve(s->cg_run(s->y, s->sigma, pred + 1, &pred));
         MAZE_HIP(hipMemcpy(x, s->y, s->G * sizeof(double), hipMemcpyDeviceToHost));
-        if (onchip && !s->onchip) res = -3;
+        if (s->onchip_abandoned) res = -3;
         if (onchip == 3 && s->onchip_w.epoch != 1u) res = -4;
     }
     delete s;
@@ -416,6 +418,29 @@ int maze_test_conj_grad(const double* b, double* x, double tol, int n) {
 int maze_test_conj_grad_pb(const double* b, double* x, double tol, int n, const double* ex,
                            const double* ey, const double* ez, const double* k2) {
     return maze_test_conj_grad_form(b, x, tol, n, ex, ey, ez, k2, 1, 0);
+}
+
+// `count` cold solves in turn, the first of them starting abandoned; on_chip[k]: solve k
+// ran in one launch.  Returns the abandoned ones.
+int maze_test_onchip_pause(const double* b, double tol, int n, int count, int* on_chip) {
+    Sim* s = scratch_sim(n);
+    s->onchip_enable();
+    s->tol = tol;
+    MAZE_HIP(hipMemcpy(s->sigma, b, s->G * sizeof(double), hipMemcpyHostToDevice));
+    int pred = 32;
+    for (int k = 0; k < count; k++) {
+        if (k == 0) {
+            const unsigned int given_up = 1u << 30;
+            MAZE_HIP(hipMemcpy(s->onchip_w.ctl, &given_up, sizeof(given_up), hipMemcpyHostToDevice));
+        }
+        s->onchip_void = k == 0;
+        maze::launch_fill(s->stream, s->G, 0.0, s->y);
+        s->cg_solve(s->cg_run(s->y, s->sigma, pred + 1, &pred));
+        on_chip[k] = s->cg.onchip;
+    }
+    const int lost = (int)s->onchip_abandoned;
+    delete s;
+    return lost;
 }
 
 unsigned int maze_test_next_epoch(unsigned int epoch, unsigned int used, unsigned int span) {

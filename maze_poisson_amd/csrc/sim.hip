@@ -603,6 +603,10 @@ void Sim::onchip_enable() {
 bool Sim::onchip_next(const GridDims& d, int limit, int two) {
     // Per-kernel timing names the sweeps, so it runs them.
     if (!onchip || prof || !(two ? cg_onchip2_fits(d) : cg_onchip_fits(d))) return false;
+    if (onchip_pause > 0) {
+        onchip_pause--;
+        return false;
+    }
     const unsigned int span = 3u * (unsigned int)limit + 6u;
     onchip_w.epoch = next_epoch(onchip_w.epoch, onchip_span, span);
     if (!onchip_w.epoch) {
@@ -611,6 +615,15 @@ bool Sim::onchip_next(const GridDims& d, int limit, int two) {
     }
     onchip_span = span;
     return true;
+}
+
+void Sim::onchip_given_up() {
+    if (onchip_abandoned++ == 0)
+        std::fprintf(stderr, "maze: a CG solve waited 0.2 s for room on the GPU and was started over in "
+                             "its slower form, as are the next %ld (maze_onchip_abandoned counts these)\n",
+                     onchip_pause_next);
+    onchip_pause = onchip_pause_next;
+    onchip_pause_next = std::min(2 * onchip_pause_next, kOnchipPauseMax);
 }
 
 // With one reduction, the direction pass after update `limit` applies its stop test.
@@ -639,8 +652,11 @@ void Sim::cg_chunk() {
 int Sim::cg_finish() {
     wait_published();
     if (cg.onchip) {
-        if (!st_host->done) {  // abandoned: x is untouched, the sweeps run the solve
-            onchip = cg.onchip = 0;
+        if (st_host->done) {
+            onchip_pause_next = kOnchipPause;
+        } else {  // abandoned: x is untouched, the sweeps run the solve
+            onchip_given_up();
+            cg.onchip = 0;
             cg_start();
             cg_chunk();
             read_state();
@@ -671,10 +687,11 @@ int Sim::cg_count_solve(const GridDims& d, const PBCoef& cpb, const double* b, d
         launch_cg_onchip(stream, d, cpb, x, rbuf, pa, pbuf, st, onchip_w);
         read_state(st);
         if (st_host->done) {
+            onchip_pause_next = kOnchipPause;
             *pred = std::max(1, st_host->res);
             return st_host->res;
         }
-        onchip = 0;  // abandoned: x is untouched
+        onchip_given_up();  // x is untouched
     }
     launch_cg_reset(stream, st, 0.0, rtol, maxit, 1, 0, 0, plain);
     launch_cg_init<double>(stream, d, cpb, x, b, rbuf, st, red, nullptr, plain);

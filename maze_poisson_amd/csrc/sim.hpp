@@ -221,9 +221,16 @@ struct Sim {
     // fits (cg_onchip_fits) -- for replicas that have the GPU to themselves: the
     // launch's work-groups wait for each other, and two of them at once could
     // each hold CUs the other waits for.  Set by the single-replica ABI; the
-    // replica engine runs the sweeps (the same bits).  Cleared when a solve was
-    // abandoned (another process waits on the same GPU).
+    // replica engine runs the sweeps (the same bits).
     int onchip = 0;
+    // An abandoned solve (its work-groups were not all on the GPU for 0.2 s: other work
+    // holds CUs) runs as sweeps, and so do the next onchip_pause ones: 256, and twice as
+    // many after each further one in a row, so that what lasts costs 0.2 s ever more
+    // rarely and what has passed costs a little time once.
+    static constexpr long kOnchipPause = 256, kOnchipPauseMax = 1 << 16;
+    long onchip_pause = 0, onchip_pause_next = kOnchipPause;
+    long onchip_abandoned = 0;  // so far
+    void onchip_given_up();
     CgOnchip onchip_w{nullptr, nullptr, 1u};
     int onchip_void = 0;           // tests: the next launch starts abandoned
     unsigned int onchip_span = 0;  // epochs the last such solve may have used

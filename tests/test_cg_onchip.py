@@ -123,6 +123,19 @@ def test_abandoned_launch_falls_back(hip_raw, n, reductions):
     assert np.array_equal(xo, xs)
 
 
+# One abandoned solve is counted, and solves go on the chip again after a pause.
+@pytest.mark.gpu
+def test_abandoned_launch_is_tried_again(hip_raw, capfd):
+    b, _ = _problem(16, 5)
+    f = hip_raw.maze_test_onchip_pause
+    I = np.ctypeslib.ndpointer(dtype=np.int32, flags="C_CONTIGUOUS")
+    f.restype, f.argtypes = ctypes.c_int, [D, ctypes.c_double, ctypes.c_int, ctypes.c_int, I]
+    on_chip = np.full(260, -1, dtype=np.int32)
+    assert f(b, 1e-3 * np.abs(b).max(), 16, len(on_chip), on_chip) == 1
+    assert (on_chip[:257] == 0).all() and (on_chip[257:] == 1).all()
+    assert capfd.readouterr().err.count("waited 0.2 s") == 1
+
+
 # The first solve after the epochs have run out.
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,reductions", [(48, 1), (48, 2), (131, 2)])
