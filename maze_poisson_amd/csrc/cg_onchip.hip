@@ -44,12 +44,14 @@ namespace maze {
 namespace {
 
 using u64 = unsigned long long;
-constexpr unsigned int kPoison = 1u << 20;
+constexpr unsigned int kPoison = 1u << 10;  // over the count of arrivals
 constexpr long long kWaitTicks = 20000000;  // 0.2 s of the 100 MHz clock
 constexpr size_t kLdsMax = 160 * 1024 - 1024;
 constexpr int kThreads = 2 * kBlock;
 constexpr int kMaxWg = 256;
 constexpr int kMaxGroups = kMaxWg / kWave;
+// Marks by every thread of a launch at once neither overflow nor look like arrivals.
+static_assert(kPoison > kMaxWg && (u64)kPoison * kMaxWg * 1024 <= 0xffffffffull, "marks overflow");
 constexpr int kVals = kCg1Sums + 1;  // the sums and max|r|
 constexpr int kLine = 16;            // words per 128-byte line
 constexpr int kHalo = 8;             // in-plane halo entries per thread, at most
