@@ -285,6 +285,8 @@ int maze_test_conj_grad_pb(const double *b, double *x, double tol, int n, const 
 int maze_test_conj_grad_form(const double *b, double *x, double tol, int n, const double *eps_x,
                              const double *eps_y, const double *eps_z, const double *k2,
                              int reductions, int onchip);
+/* The pair kernel's sqrt(r2[i]) and its reciprocal. */
+void maze_test_root(const double *r2, double *r, double *ir, int n);
 /* `count` solves of b in turn, the first starting abandoned; on_chip[k]: whether solve k
  * ran in one launch.  Returns how many were abandoned. */
 int maze_test_onchip_pause(const double *b, double tol, int n, int count, int *on_chip);

@@ -420,6 +420,17 @@ int maze_test_conj_grad_pb(const double* b, double* x, double tol, int n, const 
     return maze_test_conj_grad_form(b, x, tol, n, ex, ey, ez, k2, 1, 0);
 }
 
+void maze_test_root(const double* r2, double* r, double* ir, int n) {
+    const size_t bytes = sizeof(double) * (size_t)n;
+    double* d = nullptr;
+    MAZE_HIP(hipMalloc(&d, 3 * bytes));
+    MAZE_HIP(hipMemcpy(d, r2, bytes, hipMemcpyHostToDevice));
+    maze::launch_root(nullptr, n, d, d + n, d + 2 * (size_t)n);
+    MAZE_HIP(hipMemcpy(r, d + n, bytes, hipMemcpyDeviceToHost));
+    MAZE_HIP(hipMemcpy(ir, d + 2 * (size_t)n, bytes, hipMemcpyDeviceToHost));
+    MAZE_HIP(hipFree(d));
+}
+
 // `count` cold solves in turn, the first of them starting abandoned; on_chip[k]: solve k
 // ran in one launch.  Returns the abandoned ones.
 int maze_test_onchip_pause(const double* b, double tol, int n, int count, int* on_chip) {

@@ -355,7 +355,8 @@ void launch_force_fd_kick(hipStream_t s, const PDev& p, const double* phi, doubl
 // cutoff are skipped.  Fewer work-groups than block pairs take theirs from a queue
 // (tf_beside).  32768 ions 1.94 ms, or 2.4 beside the solve (2.14 with the library's
 // root, division and rounding), 4096 41 us (56; 50 with the launch grid's lower half
-// empty), 216 10.9 us (12.6); the sums keep their order and bits.
+// empty), 216 10.9 us (12.6); the sums keep their order and, but for what root() says of
+// 1 / r, their bits.
 constexpr int kTfB = 64;
 constexpr int kTfWaves = 4;
 constexpr int kTfCus = 256;
@@ -382,10 +383,13 @@ __device__ __forceinline__ double round_away(double x) {
     return trunc(x + copysign(0.49999999999999994, x));
 }
 
-// r = sqrt(r2) and 1 / r, both rounded as by sqrt and the division, for r2 well inside
-// the normal range: Goldschmidt's iteration for the square root and half its
-// reciprocal, then one correction of each by its exact residual (P. Markstein, IBM J.
-// Res. Dev. 34 (1990)).
+// r = sqrt(r2), rounded as by sqrt, and 1 / r, rounded as by the division or, where it
+// lies within 2^-102 of the middle of two doubles (all ones and 89 other significands of
+// r, divisors of 2^j +- c with c < 16), to either of them: Goldschmidt's iteration for the
+// square root and half its reciprocal, then one correction of each by its exact residual
+// (P. Markstein, IBM J. Res. Dev. 34 (1990)).  Telling those cases apart costs 2.6 % of
+// the kernel.  What is not well inside the normal range (coincident ions, positions that
+// are not finite) takes the library's way.
 __device__ __forceinline__ void root(double r2, double& r, double& ir) {
     const double y = __builtin_amdgcn_rsq(r2);
     double g = r2 * y, q = 0.5 * y;
@@ -398,6 +402,20 @@ __device__ __forceinline__ void root(double r2, double& r, double& ir) {
     r = fma(fma(-g, g, r2), q, g);
     const double z = q + q;
     ir = fma(fma(-r, z, 1.0), z, z);
+    if (!(r2 > 1e-200 && r2 < 1e200)) {
+        r = sqrt(r2);
+        ir = 1.0 / r;
+    }
+}
+
+__global__ void k_root(int n, const double* __restrict__ r2, double* __restrict__ r,
+                       double* __restrict__ ir) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) root(r2[i], r[i], ir[i]);
+}
+
+void launch_root(hipStream_t s, int n, const double* r2, double* r, double* ir) {
+    MAZE_LAUNCH(k_root, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, n, r2, r, ir);
 }
 
 template <bool LdsTab>
@@ -478,10 +496,6 @@ __global__ __launch_bounds__(kTfB * kTfWaves) void k_tf_tiles(
             r2 += app * app;
             double r, ir;
             root(r2, r, ir);
-            if (!(r2 > 1e-200 && r2 < 1e200)) {  // coincident ions, positions not finite
-                r = sqrt(r2);
-                ir = 1.0 / r;
-            }
             ok = ok && r <= r_cut;
             const unsigned long long m = __ballot(ok);
             mi += ok;

@@ -59,6 +59,8 @@ void launch_force_fd(hipStream_t s, const PDev& p, const double* phi);
 // when it runs (work queued before the host knows whether it is due).
 void launch_force_fd_kick(hipStream_t s, const PDev& p, const double* phi, double cdt,
                           const int* gate = nullptr);
+// The pair kernel's distance and reciprocal distance of n squared distances (tests).
+void launch_root(hipStream_t s, int n, const double* r2, double* r, double* ir);
 long tf_part_doubles(int np);
 void launch_tf(hipStream_t s, const PDev& p, PScalars* ps, Reduce red);
 bool tf_beside(int n, int np);

@@ -2,7 +2,9 @@
 in seconds).  Point-wise kernels must agree bit for bit (they follow the reference's
 operation order); anything that goes through a global sum (CG scalars) agrees to
 the stated tolerances.  Every test calls the product through its C-ABI."""
+import ctypes
 import dataclasses
+from fractions import Fraction
 
 import numpy as np
 import pytest
@@ -1016,3 +1018,59 @@ def test_mg_march_bitwise_equals_tiles(hip_raw, n, march):
         assert hip_raw.maze_test_mg_up2(b, d2, e, d, n, c1, c2, tile) == 0
         up[tile] = d
     assert np.array_equal(up[0], up[march])
+
+
+def _midpoint_roots():
+    """r2 = (s^2 - c) / 2^j for 54-bit s, exact: roots within c / (2 s) of the midpoint of
+    two doubles (s from the square roots of c modulo 2^j, bit by bit)."""
+    out = []
+    for j in (54, 55, 56):
+        for c in range(1 - 8 * 40, 8 * 40, 8):
+            x = 1
+            for b in range(3, j + 1):
+                if (x * x - c) % (1 << b):
+                    x += 1 << (b - 2)
+            for s in (x, -x, x + (1 << (j - 1)), -x - (1 << (j - 1))):
+                s %= 1 << j
+                v = (s * s - c) >> j
+                if s.bit_length() == 54 and 0 < v < 1 << 53:
+                    out += [float(v), 2.0 * v]
+    return out
+
+
+def test_pair_distance_rounding(hip_raw):
+    """r of the pair kernel is the host's (IEEE) square root, 1 / r the host's quotient or,
+    where that is a tie but for 2^-102, the other one of the two doubles."""
+    g = np.random.default_rng(11)
+    # Distances whose significand is all ones, or all ones but for the last bits.
+    ones = (2.0 - 2.0 ** -52 * np.arange(1, 600)) * 2.0 ** np.arange(-4, 5)[:, None]
+    # Quotients near ties: significands that divide 2^j +- c with a 54-bit quotient.
+    near = np.array([float.fromhex(x) for x in (
+        "0x1.024a3bd98da02p+0", "0x1.0699d36aec84ep+0", "0x1.0aadc6f562fdcp+0",
+        "0x1.202c5c315a210p+0", "0x1.2e3c6a0509ca4p+0", "0x1.4877a4a0a0d04p+0",
+        "0x1.4a6fb45f5d782p+0", "0x1.755ba34be3d40p+0", "0x1.b227794e85702p+0",
+        "0x1.c23757c848820p+0", "0x1.e20adbc4078a2p+0", "0x1.ffffff8000001p+0")])
+    r = np.concatenate([ones.ravel(), near, np.exp(g.uniform(-7, 7, 200000))])
+    r2 = [r * r]
+    for _ in range(3):  # the squares' neighbours
+        r2.append(np.nextafter(r2[-1], 0.0))
+    r2.append(np.nextafter(r2[0], np.inf))
+    r2 += [np.exp(g.uniform(-14, 14, 1000000)), np.array(_midpoint_roots()),
+           np.exp(g.uniform(np.log(1e-300), np.log(1e300), 100000)),
+           np.array([0.0, 5e-324, 1e-320, 2.3e-308, 1.7e308, np.inf, np.nan])]
+    r2 = np.ascontiguousarray(np.concatenate(r2))
+    a, b = np.zeros_like(r2), np.zeros_like(r2)
+    D = np.ctypeslib.ndpointer(dtype=np.float64, flags="C_CONTIGUOUS")
+    f = hip_raw.maze_test_root
+    f.restype, f.argtypes = None, [D, D, D, ctypes.c_int]
+    f(r2, a, b, r2.size)
+    with np.errstate(divide="ignore"):
+        root = np.sqrt(r2)
+        want = 1.0 / root
+    assert np.array_equal(a, root, equal_nan=True)
+    off = np.flatnonzero(~((b == want) | (np.isnan(b) & np.isnan(want))))
+    assert not np.isin(off, np.arange(r2.size - 7, r2.size)).any()
+    for got, q, x in zip(b[off].tolist(), want[off].tolist(), root[off].tolist()):
+        assert got in (np.nextafter(q, 0.0), np.nextafter(q, np.inf))
+        tie = (Fraction(got) + Fraction(q)) / 2
+        assert abs(tie * Fraction(x) - 1) < Fraction(1, 2 ** 102)
