@@ -431,6 +431,10 @@ void maze_test_root(const double* r2, double* r, double* ir, int n) {
     MAZE_HIP(hipFree(d));
 }
 
+int maze_test_tf_work_groups(int n, int np, int beside) {
+    return maze::tf_work_groups(n, np, beside != 0);
+}
+
 // `count` cold solves in turn, the first of them starting abandoned; on_chip[k]: solve k
 // ran in one launch.  Returns the abandoned ones.
 int maze_test_onchip_pause(const double* b, double tol, int n, int count, int* on_chip) {

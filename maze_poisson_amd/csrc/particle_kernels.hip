@@ -622,20 +622,26 @@ long tf_part_doubles(int np) {
 // takes 156 ms (166 with all work-groups at once, 162 with three per CU), of 21952 on
 // 224^3 256 (255), of 13824 on 192^3 152 (152).  Not where the pairs outlast the solve
 // (32768 ions on 128^3: 110 against 104 ms), where they are few (8000 ions: 118.3
-// against 117.2), or on grids whose CG solves take all CUs for themselves.
+// against 117.2), or on grids whose CG solves take all CUs for themselves, and never
+// where the kernel runs by itself (32768 ions: 2.08 ms, 1.70 with all work-groups).
 bool tf_beside(int n, int np) {
     const int nb = tf_blocks(np), items = tf_item(nb, nb, nb);
     return (long)n * n * n >= 64L * items && items >= 64 * kTfCus &&
            !cg_onchip2_fits(grid_dims_for(n));
 }
 
-void launch_tf(hipStream_t s, const PDev& p, PScalars* ps, Reduce red) {
+int tf_work_groups(int n, int np, bool beside) {
+    const int nb = tf_blocks(np), items = tf_item(nb, nb, nb);
+    return beside && tf_beside(n, np) ? 2 * kTfCus : items;
+}
+
+void launch_tf(hipStream_t s, const PDev& p, PScalars* ps, Reduce red, bool beside) {
     if (p.np == 0) {
         launch_sum_scaled(s, 0, 0.5, p.eion, &ps->pe_tf, red);
         return;
     }
-    const int nb = tf_blocks(p.np), items = tf_item(nb, nb, nb);
-    const dim3 g(tf_beside(p.n, p.np) ? 2 * kTfCus : items), b(kTfB * kTfWaves);
+    const int nb = tf_blocks(p.np);
+    const dim3 g(tf_work_groups(p.n, p.np, beside)), b(kTfB * kTfWaves);
     if (p.n_typ <= kTfLdsTypes)
         MAZE_LAUNCH(k_tf_tiles<true>, g, b, 0, s, p.np, p.n_typ, p.L, 1.0 / p.L, p.r_cut, p.pos,
                     p.types, p.table, p.tpart, ps->tf_queue);

@@ -834,6 +834,33 @@ def test_tf_queue_equals_grid(hip, n_p):
         assert v == out[0][0] and np.array_equal(f, out[0][1]) and np.array_equal(cnt, out[0][2])
 
 
+# The pair forces of an MD step (beside its solve, from the queue) and of a call by
+# itself (a work-group per block pair): the same bits.
+@pytest.mark.parametrize("n_p", [11649, 13824])
+def test_tf_beside_equals_alone(hip, n_p):
+    s = W.nacl_system(13824, 240, seed=3)
+    s = dataclasses.replace(s, **{k: getattr(s, k)[:n_p] for k in ("types", "pos", "vel", "mass",
+                                                                   "charges")})
+    s = dataclasses.replace(s, charges=s.charges - s.charges.mean())  # neutral
+    items = (n_p + 63) // 64 * ((n_p + 63) // 64 + 1) // 2
+    groups = hip.lib.maze_test_tf_work_groups
+    assert groups(240, n_p, 0) == items and groups(240, n_p, 1) < items
+    driver.initialize(hip, s, driver.RunConfig(tol=1.0))
+    hip.solver_set_precision(2)
+    driver.bootstrap(hip)
+    out = []
+    for step in (True, False, True, False):
+        hip.solver_md_loop_iter() if step else hip.solver_compute_forces_noel()
+        f, cnt = np.zeros((n_p, 3)), np.zeros(n_p, dtype=np.int32)
+        hip.get_fcs_noel(f)
+        hip.get_tf_neighbor_counts(cnt)
+        out.append((f, cnt))
+    hip.solver_finalize()
+    assert np.abs(out[0][0]).max() > 0 and not np.array_equal(out[0][0], out[2][0])
+    for k in (0, 2):
+        assert np.array_equal(out[k][0], out[k + 1][0]) and np.array_equal(out[k][1], out[k + 1][1])
+
+
 # ---- Poisson-Boltzmann boundary from ion radii -------------------------------------
 
 PB_RADII_SYSTEMS = {
