@@ -285,8 +285,8 @@ int maze_test_conj_grad_pb(const double *b, double *x, double tol, int n, const 
 int maze_test_conj_grad_form(const double *b, double *x, double tol, int n, const double *eps_x,
                              const double *eps_y, const double *eps_z, const double *k2,
                              int reductions, int onchip);
-/* Work-groups of the pair kernel for np ions on an n^3 grid, by itself or beside a field
- * solve. */
+/* Work-groups of the pair kernel for np ions on an n^3 grid and 256 CUs, by itself or
+ * beside a multigrid-PCG solve. */
 int maze_test_tf_work_groups(int n, int np, int beside);
 /* The pair kernel's sqrt(r2[i]) and its reciprocal. */
 void maze_test_root(const double *r2, double *r, double *ir, int n);

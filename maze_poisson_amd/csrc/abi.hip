@@ -432,7 +432,7 @@ void maze_test_root(const double* r2, double* r, double* ir, int n) {
 }
 
 int maze_test_tf_work_groups(int n, int np, int beside) {
-    return maze::tf_work_groups(n, np, beside != 0);
+    return maze::tf_work_groups(n, np, beside && Sim::tf_room(n, true, false), 256);
 }
 
 // `count` cold solves in turn, the first of them starting abandoned; on_chip[k]: solve k

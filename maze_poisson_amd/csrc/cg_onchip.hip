@@ -1280,12 +1280,7 @@ size_t lds_bytes(const GridDims& d) {
 
 int groups_of(const GridDims& d) { return (d.chunks + 1) / 2; }
 
-int compute_units() {
-    int dev = 0, cus = 0;
-    MAZE_HIP(hipGetDevice(&dev));
-    MAZE_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    return cus < kMaxWg ? cus : kMaxWg;
-}
+int work_groups() { return std::min(compute_units(), kMaxWg); }
 
 // Halo entries a thread of k_cg_onchip / k_cg_onchip2 holds, at most.
 int held(int slab) {
@@ -1365,6 +1360,13 @@ void launch_any(hipStream_t s, const OnchipArgs& a, const PBCoef& pb, double* x,
 
 }  // namespace
 
+int compute_units() {
+    int dev = 0, cus = 0;
+    MAZE_HIP(hipGetDevice(&dev));
+    MAZE_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    return cus;
+}
+
 // The vectors of a work-group's share fit it.
 static bool share_fits(const GridDims& d) {
     return d.slab <= 16 && groups_of(d) * d.slabs <= kMaxWg && lds_bytes(d) <= kLdsMax &&
@@ -1383,7 +1385,7 @@ GridDims cg_dims_for(int n) {
 }
 
 bool cg_onchip_fits(const GridDims& d) {
-    return share_fits(d) && groups_of(d) * d.slabs <= compute_units();
+    return share_fits(d) && groups_of(d) * d.slabs <= work_groups();
 }
 
 long cg_onchip_words() { return kSlot * (kMaxWg + kMaxGroups); }
@@ -1404,7 +1406,7 @@ void launch_cg_onchip(hipStream_t s, const GridDims& d, const PBCoef& pb, double
 }
 
 bool cg_onchip2_fits(const GridDims& d) {
-    const int cus = compute_units();
+    const int cus = work_groups();
     return tiles_per_wg(d, cus) > 0 || stream_slabs(d, cus) > 0;
 }
 
@@ -1412,12 +1414,12 @@ void launch_cg_onchip2(hipStream_t s, const GridDims& d, const PBCoef& pb, doubl
                        double* h, double* xs, CGState* st, const CgOnchip& w) {
     Onchip2Args a;
     a.d = d;
-    a.T = tiles_per_wg(d, compute_units());
+    a.T = tiles_per_wg(d, work_groups());
     if (!a.T) {
         StreamArgs b;
         b.d = d;
         b.groups = groups_of(d);
-        b.slabs = stream_slabs(d, compute_units());
+        b.slabs = stream_slabs(d, work_groups());
         b.nwg = b.groups * b.slabs;
         b.words = w.words;
         b.h = h;

@@ -214,10 +214,10 @@ struct Engine {
     // pairs beyond those of the replicas that ever ran at once.
     // A lane's two streams so mostly share a queue: its pair forces run between its
     // solves, beside those of others (32 replicas 283 ms; 290 with the pair forces of
-    // one replica on the queue of another's solve).  A replica whose pair kernel is
-    // made to run beside its own solve (`wide`, tf_beside) takes two streams made one
-    // right after the other, which go to different queues: 32768 ions on 256^3 153 ms
-    // for 40 steps, 188 on one queue.
+    // one replica on the queue of another's solve).  A replica with many pairs and a
+    // longer solve (`wide`, tf_overlaps) takes two streams made one right after the other,
+    // which go to different queues: 32768 ions on 256^3 153 ms for 40 steps, 188 on one
+    // queue.
     // `created` gets the drop of free device memory over a new batch: the
     // runtime sets up its hardware queues (a per-process cost, at most four
     // queues) as the first streams are made, so it is not a per-replica cost.
@@ -263,7 +263,7 @@ struct Engine {
         r.used_precision = precision_for(r.n, r.precision, r.ph);
         // Its lane comes from the pool, created four at a time and counted apart
         // from the replica's own memory.
-        r.lane = take_lane(r.stream_bytes, tf_beside(r.n, r.np));
+        r.lane = take_lane(r.stream_bytes, tf_overlaps(r.n, r.np));
         size_t free0 = 0, total = 0;
         MAZE_HIP(hipMemGetInfo(&free0, &total));
         r.arena = std::make_unique<DevArena>();

@@ -88,6 +88,9 @@ struct Reduce {
 // sized for about 512 work-groups per sweep); every replica uses it.
 GridDims grid_dims_for(int n);
 
+// CUs of the calling thread's device.
+int compute_units();
+
 // ---- launchers (grid_kernels.hip) ----------------------------------------
 void launch_laplace(hipStream_t s, const GridDims& d, const PBCoef& pb, const double* u, double* out);
 void launch_pred_sigma(hipStream_t s, const GridDims& d, const PBCoef& pb, const double* phi,

@@ -6,6 +6,8 @@
 // library/src/integrator_ovrvo.c:45-123) so that per-ion results match the
 // CPU oracle bit for bit wherever no transcendental function is involved.
 
+#include <algorithm>
+
 #include "grid.hpp"
 #include "particles.hpp"
 
@@ -353,13 +355,14 @@ void launch_force_fd_kick(hipStream_t s, const PDev& p, const double* phi, doubl
 // coefficients formed once, LDS adds without a return, pairs counted in ballots, no
 // bounds checks in full blocks.  Blocks whose extents lie further apart than the
 // cutoff are skipped.  Fewer work-groups than block pairs take theirs from a queue
-// (tf_beside).  32768 ions 1.94 ms, or 2.4 beside the solve (2.14 with the library's
+// (tf_work_groups).  32768 ions 1.94 ms, or 2.4 beside the solve (2.14 with the library's
 // root, division and rounding), 4096 41 us (56; 50 with the launch grid's lower half
 // empty), 216 10.9 us (12.6); the sums keep their order and, but for what root() says of
 // 1 / r, their bits.
 constexpr int kTfB = 64;
 constexpr int kTfWaves = 4;
-constexpr int kTfCus = 256;
+constexpr int kTfMany = 1 << 14;    // block pairs, 64 per CU
+constexpr int kTfRoomGrid = 240;
 
 __host__ __device__ __forceinline__ int tf_item(int I, int J, int nb) { return I * nb - I * (I - 1) / 2 + (J - I); }
 
@@ -614,34 +617,36 @@ long tf_part_doubles(int np) {
     return nb * (nb + 1) / 2 * 5 * 2 * kTfB;
 }
 
-// Whether the pair kernel leaves room for a solve that it runs beside and that
-// outlasts it.  With a work-group per block pair, the large tiles of the multigrid
+// Whether a solve outlasts the pairs it runs beside, and they are many: such a replica's
+// pair kernel and solve go to hardware queues of their own (the replica engine's lanes:
+// 2 to 6 % of a request from 12000 ions on 112^3 to 32768 on 256^3).
+bool tf_overlaps(int n, int np) {
+    const int nb = tf_blocks(np), items = tf_item(nb, nb, nb);
+    return (long)n * n * n >= 64L * items && items >= kTfMany;
+}
+
+// The pair kernel's work-groups, `room`: beside a solve whose kernels need room (Sim::
+// tf_room).  With a work-group per block pair, the large tiles of the finest multigrid
 // levels find no CU with enough free registers and LDS until the last pairs are out
 // (1.03 ms for a 13 us kernel at 256^3); two work-groups per CU that take pairs from a
-// queue cost the pair kernel itself a quarter.  A 40-step run of 32768 ions on 256^3
-// takes 156 ms (166 with all work-groups at once, 162 with three per CU), of 21952 on
-// 224^3 256 (255), of 13824 on 192^3 152 (152).  Not where the pairs outlast the solve
-// (32768 ions on 128^3: 110 against 104 ms), where they are few (8000 ions: 118.3
-// against 117.2), or on grids whose CG solves take all CUs for themselves, and never
-// where the kernel runs by itself (32768 ions: 2.08 ms, 1.70 with all work-groups).
-bool tf_beside(int n, int np) {
+// queue cost the pair kernel itself a quarter (32768 ions alone 2.08 ms, 1.70 with all).
+// 40 steps of 32768 ions on 256^3 take 156 ms (166 with all work-groups at once, 162 with
+// three per CU); the lines are where both measured the same: 20000 ions on 208^3 41.3 ms
+// for 15 steps (41.3), 21952 on 224^3 58.0 for 20 (57.6), 27000 on 240^3 63.0 (63.3),
+// 32768 there 71.9 (74.3), 40000 on 256^3 85 (90), 48000 on 288^3 131 (140).  Not where the
+// pairs outlast the solve (32768 ions on 128^3: 110 against 104 ms) or are few.
+int tf_work_groups(int n, int np, bool room, int cus) {
     const int nb = tf_blocks(np), items = tf_item(nb, nb, nb);
-    return (long)n * n * n >= 64L * items && items >= 64 * kTfCus &&
-           !cg_onchip2_fits(grid_dims_for(n));
+    return room && n >= kTfRoomGrid && tf_overlaps(n, np) ? std::min(2 * cus, items) : items;
 }
 
-int tf_work_groups(int n, int np, bool beside) {
-    const int nb = tf_blocks(np), items = tf_item(nb, nb, nb);
-    return beside && tf_beside(n, np) ? 2 * kTfCus : items;
-}
-
-void launch_tf(hipStream_t s, const PDev& p, PScalars* ps, Reduce red, bool beside) {
+void launch_tf(hipStream_t s, const PDev& p, PScalars* ps, Reduce red, bool room) {
     if (p.np == 0) {
         launch_sum_scaled(s, 0, 0.5, p.eion, &ps->pe_tf, red);
         return;
     }
     const int nb = tf_blocks(p.np);
-    const dim3 g(tf_work_groups(p.n, p.np, beside)), b(kTfB * kTfWaves);
+    const dim3 g(tf_work_groups(p.n, p.np, room, room ? compute_units() : 0)), b(kTfB * kTfWaves);
     if (p.n_typ <= kTfLdsTypes)
         MAZE_LAUNCH(k_tf_tiles<true>, g, b, 0, s, p.np, p.n_typ, p.L, 1.0 / p.L, p.r_cut, p.pos,
                     p.types, p.table, p.tpart, ps->tf_queue);

@@ -62,10 +62,10 @@ void launch_force_fd_kick(hipStream_t s, const PDev& p, const double* phi, doubl
 // The pair kernel's distance and reciprocal distance of n squared distances (tests).
 void launch_root(hipStream_t s, int n, const double* r2, double* r, double* ir);
 long tf_part_doubles(int np);
-// beside: a field solve runs at the same time.
-void launch_tf(hipStream_t s, const PDev& p, PScalars* ps, Reduce red, bool beside = false);
-int tf_work_groups(int n, int np, bool beside);
-bool tf_beside(int n, int np);
+// room: a field solve that needs it runs at the same time.
+void launch_tf(hipStream_t s, const PDev& p, PScalars* ps, Reduce red, bool room = false);
+int tf_work_groups(int n, int np, bool room, int cus);
+bool tf_overlaps(int n, int np);
 // F_tot = F_elec + F_noel (+ the PB boundary forces fdb, fib, fnp when given).
 void launch_force_total(hipStream_t s, const PDev& p, const double* fdb = nullptr,
                         const double* fib = nullptr, const double* fnp = nullptr);

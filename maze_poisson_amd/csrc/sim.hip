@@ -1712,7 +1712,9 @@ void Sim::step_issue() {
     auto issue_tf = [&] {
         MAZE_HIP(hipEventRecord(ev_pos, stream));
         MAZE_HIP(hipStreamWaitEvent(side, ev_pos, 0));
-        timed(kTTf, 0, [&] { launch_tf(side, p, ps, red_side, true); });
+        const bool alone = use_direct() || (onchip && c_rhs);
+        const bool room = tf_room(n, precision == kMixedMG && !pb, alone, mg_stop);
+        timed(kTTf, 0, [&] { launch_tf(side, p, ps, red_side, room); });
         MAZE_HIP(hipEventRecord(ev_tf, side));
     };
     if (step_tf && !tf_late) issue_tf();

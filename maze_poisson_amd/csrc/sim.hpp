@@ -274,6 +274,18 @@ struct Sim {
     Reduce red_side{};
     int tf_overlap = 1;
     int tf_late = 1;
+    // Whether a step's pair kernel leaves room for its solve (tf_work_groups).  A mixed
+    // multigrid cycle gains by it while its coarsest level is one work-group's; an odd one
+    // above 16^3, of several kernels of many work-groups, loses more to pairs that last
+    // longer (30000 ions on 248^3 91 against 85 ms for 20 steps, 48000 on 304^3 177
+    // against 161 for 15).  Not beside the direct solve (2.74 against 2.69 ms a step at
+    // 256^3), whose passes fill the chip, or a coarse CG that waits for the whole chip.
+    // FP64, MIXED-CG and PB steps gain 1 to 2 % at 256^3.
+    static bool tf_room(int n, bool mixed_mg, bool alone, int mg_stop = default_mg_stop()) {
+        if (alone) return false;
+        const std::vector<int> sizes = mixed_mg ? mg_sizes(n, mg_stop) : std::vector<int>();
+        return sizes.empty() || sizes.back() <= kMgCoarseLds;
+    }
 
     double* dscalar = nullptr;  // device scratch scalar
     double* hscalar = nullptr;  // pinned

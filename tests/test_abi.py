@@ -80,3 +80,16 @@ def test_reference_abi_fixture_is_current():
     mg = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(mg)
     assert mg.abi_fixture() == REF_ABI
+
+
+def test_pair_kernel_work_groups(hip):
+    """A work-group per pair of 64-ion blocks, but two per CU beside the multigrid solves
+    that gain by it: large grids whose coarsest level is at most 16^3."""
+    f = hip.lib.maze_test_tf_work_groups
+    items = lambda n_p: (n_p + 63) // 64 * ((n_p + 63) // 64 + 1) // 2
+    for n_p, n in ((27000, 240), (32768, 256), (40000, 256), (48000, 288), (11649, 240)):
+        assert f(n, n_p, 1) == 512 and f(n, n_p, 0) == items(n_p)
+    for n_p, n in ((216, 48), (12000, 128), (16000, 150), (20000, 156), (20000, 160),
+                   (21952, 224), (24000, 232), (30000, 248), (36000, 264), (38000, 272),
+                   (48000, 304), (48000, 256), (11000, 240), (0, 32)):
+        assert f(n, n_p, 1) == f(n, n_p, 0) == items(n_p)
