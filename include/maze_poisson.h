@@ -278,7 +278,7 @@ int maze_test_conj_grad(const double *b, double *x, double tol, int n);
 int maze_test_conj_grad_pb(const double *b, double *x, double tol, int n, const double *eps_x,
                            const double *eps_y, const double *eps_z, const double *k2);
 /* The same solves (ex == NULL: Poisson) with one or two reductions per
- * iteration, as sweeps (onchip 0) or as one launch with the CG vectors on the
+ * iteration (0: as the FP64 modes choose), as sweeps (onchip 0) or as one launch with the CG vectors on the
  * chip (bit-identical; -2 if the grid does not fit it, -3 if the launch was
  * abandoned and the sweeps ran; onchip 2: it starts abandoned; onchip 3: the epochs
  * start anew with it, -4 if they do not). */

@@ -383,26 +383,29 @@ int maze_test_conj_grad_form(const double* b, double* x, double tol, int n, cons
         s->init_pb(0.0, 0.0);
         s->set_eps_k2(ex, ey, ez, k2);
     }
-    s->precision = reductions == 2 ? maze::kMixedMG : maze::kFP64;
     s->tol = tol;
-    int res = -2;
-    if (!onchip || (s->cg_two() ? maze::cg_onchip2_fits(s->dims) : maze::cg_onchip_fits(s->cgd))) {
+    int res = -2, pred = 32;
+    Sim::CgRun run = s->cg_run(s->y, s->sigma, pred + 1, &pred);
+    if (reductions) {
+        run.two = reductions == 2;
+        run.d = run.two ? s->dims : s->cgd;
+    }
+    if (!onchip || (run.two ? maze::cg_onchip2_fits(run.d) : maze::cg_onchip_fits(run.d))) {
         MAZE_HIP(hipMemcpy(s->sigma, b, s->G * sizeof(double), hipMemcpyHostToDevice));
         MAZE_HIP(hipMemcpy(s->y, x, s->G * sizeof(double), hipMemcpyHostToDevice));
-        int pred = 32;
         if (onchip == 3) {  // after a solve with the last epochs there are
-            s->onchip_next(s->cg_two() ? s->dims : s->cgd, n * n, s->cg_two());
+            s->onchip_next(run.d, n * n, run.two);
             s->onchip_w.epoch = 0xffffffffu - 2 * s->onchip_span;
-            s->cg_solve(s->cg_run(s->y, s->sigma, pred + 1, &pred));
+            s->cg_solve(run);
             MAZE_HIP(hipMemcpy(s->y, x, s->G * sizeof(double), hipMemcpyHostToDevice));
         }
         if (onchip == 2) {
-            s->onchip_next(s->cg_two() ? s->dims : s->cgd, n * n, s->cg_two());
+            s->onchip_next(run.d, n * n, run.two);
             const unsigned int given_up = 1u << 30;
             MAZE_HIP(hipMemcpy(s->onchip_w.ctl, &given_up, sizeof(given_up), hipMemcpyHostToDevice));
             s->onchip_void = 1;
         }
-        res = s->cg_solve(s->cg_run(s->y, s->sigma, pred + 1, &pred));
+        res = s->cg_solve(run);
         MAZE_HIP(hipMemcpy(x, s->y, s->G * sizeof(double), hipMemcpyDeviceToHost));
         if (s->onchip_abandoned) res = -3;
         if (onchip == 3 && s->onchip_w.epoch != 1u) res = -4;
@@ -412,12 +415,12 @@ int maze_test_conj_grad_form(const double* b, double* x, double tol, int n, cons
 }
 
 int maze_test_conj_grad(const double* b, double* x, double tol, int n) {
-    return maze_test_conj_grad_form(b, x, tol, n, nullptr, nullptr, nullptr, nullptr, 1, 0);
+    return maze_test_conj_grad_form(b, x, tol, n, nullptr, nullptr, nullptr, nullptr, 0, 0);
 }
 
 int maze_test_conj_grad_pb(const double* b, double* x, double tol, int n, const double* ex,
                            const double* ey, const double* ez, const double* k2) {
-    return maze_test_conj_grad_form(b, x, tol, n, ex, ey, ez, k2, 1, 0);
+    return maze_test_conj_grad_form(b, x, tol, n, ex, ey, ez, k2, 0, 0);
 }
 
 void maze_test_root(const double* r2, double* r, double* ir, int n) {

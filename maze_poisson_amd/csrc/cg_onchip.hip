@@ -1373,6 +1373,8 @@ static bool share_fits(const GridDims& d) {
            2 * d.n * d.slab <= held(d.slab) * kThreads;
 }
 
+bool cg_one_reduction(const GridDims& d) { return share_fits(d); }
+
 // The flattest slabs that leave at most one work-group per CU, where the grid
 // then fits (up to 128^3).
 GridDims cg_dims_for(int n) {

@@ -155,8 +155,10 @@ inline unsigned int next_epoch(unsigned int epoch, unsigned int used, unsigned i
     const unsigned long long e = (unsigned long long)epoch + used;
     return e + span <= 0xffffffffull ? (unsigned int)e : 0u;
 }
-// The launch shape of FP64 CG on an n^3 grid, in either form.
+// The launch shape of FP64 CG on an n^3 grid, in either form, and whether it runs with
+// one reduction per iteration.
 GridDims cg_dims_for(int n);
+bool cg_one_reduction(const GridDims& d);
 bool cg_onchip_fits(const GridDims& d);
 // launch_cg_dir / launch_cg_update's solve (two reductions an iteration) likewise,
 // h, xs: scratch grids; three times the epochs.

@@ -681,7 +681,8 @@ int Sim::cg_count_solve(const GridDims& d, const PBCoef& cpb, const double* b, d
                         double rtol, int maxit, double* rbuf, double* pa, double* pbuf, int* pred,
                         CGState* st) {
     const int plain = cpb.ex ? 1 : 0;
-    if (onchip_next(d, maxit)) {
+    const int two = cg_one_reduction(d) ? 0 : 1, last = maxit + (two ? 0 : 1);
+    if (!two && onchip_next(d, maxit)) {
         launch_cg_reset(stream, st, 0.0, rtol, maxit, 1, 0, 0, plain, onchip_w.ctl);
         launch_cg_init<double>(stream, d, cpb, x, b, rbuf, st, red, nullptr, plain);
         launch_cg_onchip(stream, d, cpb, x, rbuf, pa, pbuf, st, onchip_w);
@@ -700,13 +701,18 @@ int Sim::cg_count_solve(const GridDims& d, const PBCoef& cpb, const double* b, d
     double* pin = pa;
     double* pout = pbuf;
     for (;;) {
-        for (int c = 0; c < chunk && launched <= maxit; c++, launched++) {
-            launch_cg1_dir(stream, d, cpb, pin, rbuf, pout, st, red, launched == 0);
-            launch_cg1_update(stream, d, cpb, pout, x, rbuf, st);
+        for (int c = 0; c < chunk && launched < last; c++, launched++) {
+            if (two) {
+                launch_cg_dir<double>(stream, d, cpb, pin, rbuf, pout, st, red, launched == 0);
+                launch_cg_update<double>(stream, d, cpb, pout, x, rbuf, st, red);
+            } else {
+                launch_cg1_dir(stream, d, cpb, pin, rbuf, pout, st, red, launched == 0);
+                launch_cg1_update(stream, d, cpb, pout, x, rbuf, st);
+            }
             std::swap(pin, pout);
         }
         read_state(st);
-        if (st_host->done || launched > maxit) break;
+        if (st_host->done || launched >= last) break;
         chunk = std::max(4, chunk / 4);
     }
     *pred = std::max(1, st_host->res);

@@ -237,11 +237,16 @@ struct Sim {
     void onchip_enable();  // right after the constructor
     // Whether the next solve on grid d goes on the chip (sets its exchange up).
     bool onchip_next(const GridDims& d, int limit, int two = 0);
-    // FP64 CG runs with one reduction per iteration (Cg1) in the FP64 precisions.
+    // FP64 CG runs with one reduction per iteration (Cg1) in the FP64 precisions, on grids
+    // whose vectors fit the chip: as sweeps, on larger ones, it takes up to 5 % longer than
+    // two (a step of 8000 ions on 160^3 5.76 against 5.47 ms, of 4096 on 131^3 3.06 against
+    // 3.00; 4096 on 128^3 in the replica engine 52.8 against 54.9 ms for 10).
     // The mixed ones' cold solves keep two: an FP32 inner solve turns a last-bit
     // difference of its start into 2.6e-9 of the forces after 200 steps (4096
     // ions / 128^3), so those trajectories stay, bit for bit, what they were.
-    bool cg_two() const { return precision == kMixedCG || precision == kMixedMG; }
+    bool cg_two() const {
+        return precision == kMixedCG || precision == kMixedMG || !cg_one_reduction(cgd);
+    }
     CgRun cg_run(double* x, const double* b, int chunk, int* pred) const {
         return CgRun{cg_two() ? dims : cgd, pbc(), x, r, p0, p1, n * n, 0, chunk, pred, b, tol,
                      cg_two() ? 1 : 0, 0};

@@ -123,6 +123,21 @@ def test_abandoned_launch_falls_back(hip_raw, n, reductions):
     assert np.array_equal(xo, xs)
 
 
+# FP64 solves run with one reduction per iteration where their vectors fit the chip, else
+# with two, which as sweeps are the faster ones.
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,reductions", [(64, 1), (FIT_MAX, 1), (FIT_MAX + 1, 2), (136, 2)])
+def test_fp64_reductions(hip_raw, n, reductions):
+    b, x0 = _problem(n, 6)
+    tol = 1e-4 * np.abs(b).max()
+    x, xr = x0.copy(), x0.copy()
+    assert hip_raw.maze_test_conj_grad(b, x, tol, n) == _solve(hip_raw, b, xr, tol, n, reductions, 0)
+    assert np.array_equal(x, xr)
+    xr = x0.copy()
+    _solve(hip_raw, b, xr, tol, n, 3 - reductions, 0)
+    assert not np.array_equal(x, xr)
+
+
 # One abandoned solve is counted, and solves go on the chip again after a pause.
 @pytest.mark.gpu
 def test_abandoned_launch_is_tried_again(hip_raw, capfd):
