@@ -253,9 +253,11 @@ void get_neighbors(int64_t *recv);
 /* Number of partners within the Tosi-Fumi cutoff per ion, int32[n_p]. */
 void get_tf_neighbor_counts(int *recv);
 
-/* Per-kernel timing with HIP events on the replica's stream (only solver
- * iterations that did work are counted).  Names: "cg_dir", "cg_update",
- * "cg_dir_f32", "cg_update_f32". */
+/* Per-kernel timing with HIP events on the replica's streams (only solver
+ * iterations that did work are counted).  Names: "cg_dir", "cg_update" (FP64 CG as
+ * sweeps), "cg_onchip" (a whole FP64 CG solve in one launch), "cg_dir_f32",
+ * "cg_update_f32", "mg_down_l0", "mg_up_l0", "refine", "pred_sigma", "tf_pairs",
+ * "cic", "pb_maps", "pb_forces". */
 void maze_prof_enable(int on);
 void maze_prof_reset(void);
 int maze_prof_get(const char *name, double *total_ms, long *count);

@@ -579,10 +579,15 @@ void Sim::cg_issue(const CgRun& c) {
     cg_start();
     if (!cg.onchip)
         cg_chunk();
-    else if (cg.two)
-        launch_cg_onchip2(stream, cg.d, cg.pbc, cg.x, cg.rbuf, cg.pin, cg.pout, st, onchip_w);
     else
-        launch_cg_onchip(stream, cg.d, cg.pbc, cg.x, cg.rbuf, cg.pin, cg.pout, st, onchip_w);
+        timed(kTCgOnchip, 0, [&] {
+            if (cg.two)
+                launch_cg_onchip2(stream, cg.d, cg.pbc, cg.x, cg.rbuf, cg.pin, cg.pout, st,
+                                  onchip_w);
+            else
+                launch_cg_onchip(stream, cg.d, cg.pbc, cg.x, cg.rbuf, cg.pin, cg.pout, st,
+                                 onchip_w);
+        });
     publish();
 }
 
@@ -601,8 +606,7 @@ void Sim::onchip_enable() {
 }
 
 bool Sim::onchip_next(const GridDims& d, int limit, int two) {
-    // Per-kernel timing names the sweeps, so it runs them.
-    if (!onchip || prof || !(two ? cg_onchip2_fits(d) : cg_onchip_fits(d))) return false;
+    if (!onchip || !(two ? cg_onchip2_fits(d) : cg_onchip_fits(d))) return false;
     if (onchip_pause > 0) {
         onchip_pause--;
         return false;

@@ -138,6 +138,31 @@ def test_fp64_reductions(hip_raw, n, reductions):
     assert not np.array_equal(x, xr)
 
 
+# Per-kernel timing times the kernels of a run without it.
+@pytest.mark.gpu
+def test_timing_keeps_the_path(hip, hip_raw):
+    s = W.nacl_system(216, 32, seed=1)
+    out = []
+    for timing in (0, 1):
+        driver.initialize(hip, s, driver.RunConfig(tol=W.poisson_tol(s)))
+        driver.bootstrap(hip)
+        hip_raw.maze_prof_reset()
+        hip_raw.maze_prof_enable(timing)
+        for _ in range(3):
+            hip.solver_md_loop_iter()
+        count = {}
+        for name in ("cg_onchip", "cg_dir", "cg_update"):
+            ms, k = ctypes.c_double(), ctypes.c_long()
+            assert hip_raw.maze_prof_get(name.encode(), ctypes.byref(ms), ctypes.byref(k)) == 0
+            count[name] = k.value
+            assert (ms.value > 0) == (k.value > 0)
+        hip_raw.maze_prof_enable(0)
+        assert count == {"cg_onchip": 3 * timing, "cg_dir": 0, "cg_update": 0}
+        out.append(driver.snapshot(hip, s)["fcs_tot"])
+        hip.solver_finalize()
+    assert np.array_equal(out[0], out[1])
+
+
 # One abandoned solve is counted, and solves go on the chip again after a pause.
 @pytest.mark.gpu
 def test_abandoned_launch_is_tried_again(hip_raw, capfd):
