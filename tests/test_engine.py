@@ -244,3 +244,32 @@ def test_engine_physics_rejects_invalid(hip):
             assert e.request_stats(other)["steps"] == 0
             with pytest.raises(RuntimeError):
                 e.result(other)
+
+
+@pytest.mark.parametrize("mixed_init", [True, False])
+def test_engine_direct_solves(hip, mixed_init):
+    """Replicas at a tolerance that the mixed mode meets by the direct solve, alone and
+    among others that iterate, on one thread (with graphs) and three: the bits of the
+    single-replica path, and every array from the arena."""
+    ss = systems()[:3]
+    refs = []
+    for s in ss:
+        driver.initialize(hip, s, driver.RunConfig(tol=W.poisson_tol(s, 1e-10)))
+        hip.lib.solver_set_precision(2)
+        hip.lib.solver_set_mixed_init(1 if mixed_init else 0)
+        driver.bootstrap(hip)
+        for _ in range(STEPS):
+            hip.solver_md_loop_iter()
+        refs.append(driver.snapshot(hip, s, fields=False))
+        hip.solver_finalize()
+    for others, threads in ((0, 1), (4, 1), (4, 3)):
+        with ReplicaEngine(hip, max_slots=8, threads=threads, mixed_init=mixed_init) as e:
+            ids = [e.submit(s, STEPS, tol=W.poisson_tol(s, 1e-10)) for s in ss]
+            more = [e.submit(s, STEPS + 2) for s in W.ensemble_systems(others, sizes=(216, 512),
+                                                                       seed0=4300)]
+            e.run()
+            for rid, ref in zip(ids, refs):
+                rs = e.request_stats(rid)
+                assert rs["precision"] == 2 and rs["failures"] == 0 and rs["arena_overflow"] == 0
+                assert same(e.result(rid), ref)
+            assert all(e.request_stats(r)["failures"] == 0 for r in more)
