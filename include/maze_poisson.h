@@ -262,8 +262,8 @@ void maze_prof_enable(int on);
 void maze_prof_reset(void);
 int maze_prof_get(const char *name, double *total_ms, long *count);
 int maze_grid_blocks(void);
-/* FP64 CG solves of up to 128^3 (and the cold ones of the mixed modes at some larger
- * sizes) run in one launch that needs the whole GPU.  One that waits for it in vain,
+/* FP64 CG solves of up to 129^3, and of 130 to 135, 140, 141, 143 to 146, 160 and 161
+ * points a side, run in one launch that needs the whole GPU (256 CUs).  One that waits for it in vain,
  * 0.2 s, is run again in another form (the same result), as are the next 256 or more;
  * stderr tells of the first.  How many since solver_initialize: */
 long maze_onchip_abandoned(void);

@@ -489,9 +489,10 @@ __global__ __launch_bounds__(kThreads) void k_cg_onchip(OnchipArgs A, PBCoef pb,
 
 // ---- two reductions per iteration ------------------------------------------------
 // The iteration of k_cg_dir and k_cg_update with their bits: <p, A p>, then the
-// update and <r, r>, max|r|.  For the cold solves of the mixed precisions: their
-// FP32 inner solves turn a last-bit difference of the start into 2.6e-9 of the
-// forces after 200 steps at 4096 ions / 128^3, so a trajectory stays what it was.
+// update and <r, r>, max|r|.  For FP64 modes above 128^3 (Sim::cg_two) and for the
+// cold solves of the mixed precisions: their FP32 inner solves turn a last-bit
+// difference of the start into 2.6e-9 of the forces after 200 steps at 4096 ions /
+// 128^3, so a trajectory stays what it was.
 // Two exchanges an iteration, of the sums of each tile of `march` (grid_dims_for)
 // in the order of block_sum and reduce_partials_sum; the halo is that of r.
 struct Onchip2Args {
@@ -868,12 +869,13 @@ __global__ __launch_bounds__(NT) void k_cg_onchip2(Onchip2Args A, PBCoef pb, dou
 }
 
 // ---- larger grids: x and the halo stay in memory -----------------------------------
-// The two-reduction solve of grids whose vectors do not fit whole (about 130^3 to
-// 161^3): r and A p in registers, the own p in LDS without the halo in j and i,
-// which is read from its owner's copy in memory after a third, neighbours-only
-// exchange.  x streams through memory while the sums of the second exchange are
-// on their way.  A work-group holds two tiles of one slab, of the last two slabs
-// where the last is a short one.
+// The two-reduction solve of grids whose vectors do not fit whole: r and A p in
+// registers, the own p in LDS without the halo in j and i, which is read from its
+// owner's copy in memory after a third, neighbours-only exchange.  x streams through
+// memory while the sums of the second exchange are on their way.  A work-group holds
+// two tiles of one slab, of the last two slabs where the last is a short one.  The
+// slabs are the sweeps' (the sums keep their order), so not every size fits 256 CUs:
+// 130 to 135, 140, 141, 143 to 146, 160 and 161 do, the others run as sweeps.
 //
 // An iteration moves x (16 B per point), the edges of p (10 B) and the PB
 // coefficients (32 B), where the sweeps move 64 and 128 B: at 160^3 27.6 against
@@ -930,7 +932,6 @@ __global__ __launch_bounds__(kThreads) void k_cg_stream(StreamArgs A, PBCoef pb,
     const int ip = (i1 == n ? 0 : i1) * n2 + pl;
     const bool edge = jl || jh;  // is a neighbour of other work-groups' points
     const int nb = A.d.blocks;
-    const int tiles = min(2, A.d.chunks - 2 * g0);
     const double cr = st->plain ? -1.0 : 1.0 / 6.0;
     double rdv = st->rdv;
     int iter = 0;

@@ -96,7 +96,7 @@ struct Sim {
     // The mixed multigrid mode solves directly (launch_spectral_solve) where the
     // tolerance is below kDirectRtol of the largest ion's right-hand side
     // 4 pi q / (h eps): one multigrid-PCG pass (kMgInnerRtol) then falls short, and
-    // two take 850 us a step at 4096 ions / 128^3 against 150 us.  Above it one
+    // two take 850 us a step at 4096 ions / 128^3 against 198 us.  Above it one
     // pass stops just inside the tolerance, 4e-7 from the exact forces, and
     // stays: its trajectories are to remain what they were.
     static constexpr double kDirectRtol = 1e-9;
