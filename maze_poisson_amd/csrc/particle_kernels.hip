@@ -355,10 +355,9 @@ void launch_force_fd_kick(hipStream_t s, const PDev& p, const double* phi, doubl
 // coefficients formed once, LDS adds without a return, pairs counted in ballots, no
 // bounds checks in full blocks.  Blocks whose extents lie further apart than the
 // cutoff are skipped.  Fewer work-groups than block pairs take theirs from a queue
-// (tf_work_groups).  32768 ions 1.94 ms, or 2.4 beside the solve (2.14 with the library's
-// root, division and rounding), 4096 41 us (56; 50 with the launch grid's lower half
-// empty), 216 10.9 us (12.6); the sums keep their order and, but for what root() says of
-// 1 / r, their bits.
+// (tf_work_groups).  By itself 32768 ions 1.73 ms (1.92 with the library's root, division
+// and rounding and none skipped; 2.09 from the queue), 4096 44.5 us (60), 216 11.7 us
+// (12.9); the sums keep their order and, but for what root() says of 1 / r, their bits.
 constexpr int kTfB = 64;
 constexpr int kTfWaves = 4;
 constexpr int kTfMany = 1 << 14;    // block pairs, 64 per CU
@@ -629,7 +628,7 @@ bool tf_overlaps(int n, int np) {
 // tf_room).  With a work-group per block pair, the large tiles of the finest multigrid
 // levels find no CU with enough free registers and LDS until the last pairs are out
 // (1.03 ms for a 13 us kernel at 256^3); two work-groups per CU that take pairs from a
-// queue cost the pair kernel itself a quarter (32768 ions alone 2.08 ms, 1.70 with all).
+// queue cost the pair kernel itself a fifth (32768 ions alone 2.09 ms, 1.73 with all).
 // 40 steps of 32768 ions on 256^3 take 156 ms (166 with all work-groups at once, 162 with
 // three per CU); the lines are where both measured the same: 20000 ions on 208^3 41.3 ms
 // for 15 steps (41.3), 21952 on 224^3 58.0 for 20 (57.6), 27000 on 240^3 63.0 (63.3),
